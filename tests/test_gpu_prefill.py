@@ -362,6 +362,13 @@ def test_stage_prefill_matches_oracle(wz, orc, gpu, p0, B, prefix):
         st.close()
 
 
+@pytest.mark.parametrize("p0,B,prefix", [(0, 31, 0), (0, 32, 0), (0, 33, 0), (3, 64, 3), (0, 97, 0)])
+def test_stage_prefill_at_recurrence_buffer_edges(wz, orc, gpu, p0, B, prefix):
+    """Chunks around multiples of the 32 rows the delta rule keeps in flight: no full buffer, full
+    buffers only, and both with a rest of one row."""
+    test_stage_prefill_matches_oracle(wz, orc, gpu, p0, B, prefix)
+
+
 def run_chunks(cfg, toks, splits, seed=SEED, n_ctx=0):
     st = wzy_amd.Stage(cfg)
     st.load_synthetic(seed, n_ctx)

@@ -11,8 +11,8 @@
 //                writes a block into the streams.
 //  GDN           pf_gdn_ab (gates), pf_gdn_conv (causal conv + SiLU + L2 of q/k heads over all rows
 //                at once), pf_gdn_hist (conv history), pf_gdn_recur (the delta rule, sequential over
-//                the rows: 32 lanes per state column, 4 rows each in registers, q/k staged in LDS
-//                32 steps at a time), pf_gdn_norm (gated RMS norm, bf16).
+//                the rows: 32 lanes per state column, 4 rows each in registers; k, v and gates staged in
+//                LDS 32 rows at a time, q in registers), pf_gdn_norm (gated RMS norm, bf16).
 //  QSA           pf_qsa_prep (q / k / indexer-q norms + RoPE, INT8 KV append), pf_idx_append (the
 //                indexer keys of every block the chunk completes, one workgroup per block, then
 //                pf_idx_tail), block scores on fp16 MFMA (pf_score), top-k with the decode kernel,
@@ -32,6 +32,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x3_t __attribute__((ext_vector_type(3)));
 
 namespace {
 
@@ -465,6 +466,24 @@ WZY_DEV float sum32_pl(float v) {
     asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
     return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
+// Sums of 32 per-lane values over each 32-lane half, transposed: lane r of the half returns the sum of
+// v[r].  Five partner levels, each splitting the values a lane holds in two (16 swaps + 16 adds, then
+// reduce_level's 3 operations per value left): about 2.4 operations per value instead of 7.
+WZY_DEV float sum32_t(const float (&v)[32]) {
+    const int lane = threadIdx.x & 63;
+    float b[16], c[8], d[4], e[2], f[1];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        uint32_t x = __builtin_bit_cast(uint32_t, v[i]), y = __builtin_bit_cast(uint32_t, v[i + 16]);
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+        b[i] = __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+    }
+    reduce_level<DPP_ROW_ROR8, 16, 1>(b, c, (lane & 8) != 0);
+    reduce_level<DPP_HALF_MIRROR, 8, 1>(c, d, (lane & 4) != 0);
+    reduce_level<DPP_XOR2, 4, 1>(d, e, (lane & 2) != 0);
+    reduce_level<DPP_XOR1, 2, 1>(e, f, (lane & 1) != 0);
+    return f[0];
+}
 
 constexpr int GR_LPC = 32;                    // lanes per state column (half a wave)
 constexpr int GR_RPL = 128 / GR_LPC;          // state rows per lane (4)
@@ -472,44 +491,28 @@ constexpr int GR_CPW = 64 / GR_LPC;           // columns per wave (2)
 constexpr int GR_WAVES = 4;
 constexpr int GR_COLS = GR_CPW * GR_WAVES;    // columns per workgroup (8)
 constexpr int GR_STEPS = 32;                  // rows staged per LDS buffer (= lanes per column: lane r
-                                              // keeps row r's output for one store per buffer)
-static_assert(GR_STEPS * GR_COLS <= 256, "v staging: one value per thread");
+                                              // stores row r's output)
+static_assert(GR_STEPS * GR_COLS == 256, "v staging: one value per thread");
 static_assert(GR_RPL == 4, "the row loop holds 4 state rows per lane");
 static_assert(GR_STEPS == GR_LPC, "one output row per lane of a column");
-
-// k . q per (row, key head), with the recurrence's lane layout (lane r of a 32-lane half holds
-// elements 4r .. 4r+3) and its 32-lane sum: a parallel pass, so the sequential row loop below reads
-// one value per row instead of forming and reducing the product itself.  grid ceil(B * hk / 8), 256
-// threads (8 pairs per workgroup, one per 32-lane half).
-__global__ void __launch_bounds__(256) pf_gdn_kq_kernel(PfGdn g) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, r8 = lane & 31;
-    const int np = g.B * g.hk, QKV = (2 * g.hk + g.hv) * 128;
-    const int p = blockIdx.x * 8 + w * 2 + (lane >> 5), pc = min(p, np - 1);
-    const int t = pc / g.hk, kh = pc - t * g.hk;
-    const float4 q4 = *(const float4*) (g.conv_out + (size_t) t * QKV + kh * 128 + r8 * GR_RPL);
-    const float4 k4 = *(const float4*) (g.conv_out + (size_t) t * QKV + (g.hk + kh) * 128 + r8 * GR_RPL);
-    float kq = k4.x * q4.x;
-    kq = fmaf(k4.y, q4.y, kq);
-    kq = fmaf(k4.z, q4.z, kq);
-    kq = fmaf(k4.w, q4.w, kq);
-    kq = sum32_pl(kq);
-    if (r8 == 0 && p < np) g.kq[p] = kq;
-}
 
 // Delta rule over the chunk's rows for one value head and GR_COLS state columns (each column of
 // the state evolves independently): per row, S *= decay; kv = S^T k; delta = (v - kv) * beta;
 // S += k delta^T; o = S^T q / sqrt(128).  grid (hv * 128 / GR_COLS), 256 threads.  A column's 128
-// rows are spread over 32 lanes (4 per lane), so a row costs a few instructions per lane and two
-// 32-lane sums (DPP within each 16-lane row, then a permlane swap); k . q comes precomputed.  The
-// rows' q and k (all 128 of the key head), the columns' v and the per-row scalars go through LDS 32
-// rows at a time, the next 32 loaded while these run.
+// rows are spread over 32 lanes (4 per lane), so 16 heads put one wave on every SIMD of the chip and a row
+// costs what one wave issues, serially from row to row.  Only kv is reduced over the lanes in that chain
+// (DPP within each 16-lane row, then a permlane swap); a row's S^T q stays a per-lane partial sum, and 32
+// rows of them are reduced together, transposed, when their buffer ends (2.4 operations a row instead of 9,
+// and no k . q correction).  k and, per column, v with the row's decay and beta go through LDS 32 rows at a
+// time in 16-byte pieces, the next 32 loaded while these run; q stays out of LDS.
+// 8,192 rows x 16 heads: 1,050 us with both sums reduced per row and k, q, v through LDS; 861 with the
+// transposed sum and reads two rows ahead; 784 with q in registers (about 32 instructions a row, of which
+// 13 form the chain through kv).
 // (pf_gdn_recur_kh_kernel, src/wzy_qsa_wmma.cuh:56-195; fused_gdn_step_norm_multi,
 // src/wzy_kernels_v2.cuh:908-984)
 __global__ void __launch_bounds__(256) pf_gdn_recur_kernel(PfGdn g) {
-    __shared__ __align__(16) float sq[2][GR_STEPS][128];
     __shared__ __align__(16) float sk[2][GR_STEPS][128];
-    __shared__ float sv[2][GR_STEPS][GR_COLS];
-    __shared__ float4 sgb[2][GR_STEPS];                         // per row: decay, beta, k . q, unused
+    __shared__ f32x4_t svg[2][GR_STEPS][GR_COLS];               // v, decay, beta, unused
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int h = blockIdx.x / (128 / GR_COLS), cb = blockIdx.x % (128 / GR_COLS);
     const int kh = h % g.hk;
@@ -521,100 +524,148 @@ __global__ void __launch_bounds__(256) pf_gdn_recur_kernel(PfGdn g) {
 #pragma unroll
     for (int i = 0; i < GR_RPL; ++i) s[i] = S[(size_t) (r8 * GR_RPL + i) * 128 + col];
 
-    // staging of rows t0 .. t0+GR_STEPS-1: q and k (128 each) of key head kh, v of the columns, the
-    // per-row decay, beta and k . q.  Row indices are clamped (rows past the chunk are never used), so
-    // every load is unconditional.
-    constexpr int QK_PER = GR_STEPS * 2 * 128 / 256;      // floats per thread (32)
-    float rq[QK_PER];
-    float rv = 0.f, rg = 0.f;
-    const int qk_off = (tid >= 128 ? g.hk * 128 : 0) + kh * 128 + (tid & 127);
+    // staging of rows t0 .. t0+GR_STEPS-1.  Row indices are clamped (rows past the chunk are never
+    // used), so every load is unconditional.  Thread -> 4 k values of rows tid / 32 + 8 u; v and gates
+    // of row tid / 8, column tid % 8.
+    constexpr int K_PER = GR_STEPS * 128 / 4 / 256;       // 16-byte pieces per thread (4)
+    f32x4_t rk[K_PER];
+    f32x4_t rv = {0.f, 0.f, 0.f, 0.f};
+    const int k_e = (tid & 31) * 4;
+    const float* k_p = g.conv_out + (size_t) (g.hk + kh) * 128 + k_e;
+    const float* v_p = g.conv_out + (size_t) 2 * g.hk * 128 + h * 128 + cb * GR_COLS + tid % GR_COLS;
     auto load = [&](int t0) {
 #pragma unroll
-        for (int u = 0; u < QK_PER; ++u) rq[u] = g.conv_out[(size_t) min(t0 + u, g.B - 1) * QKV + qk_off];
-        {
-            const int step = min(tid / GR_COLS, GR_STEPS - 1), j = tid % GR_COLS, t = min(t0 + step, g.B - 1);
-            rv = g.conv_out[(size_t) t * QKV + 2 * g.hk * 128 + h * 128 + cb * GR_COLS + j];
-        }
-        {
-            const int t = min(t0 + (tid & (GR_STEPS - 1)), g.B - 1);
-            const float* src = tid < GR_STEPS ? g.decay + (size_t) t * g.hv + h
-                               : tid < 2 * GR_STEPS ? g.beta + (size_t) t * g.hv + h
-                                                    : g.kq + (size_t) t * g.hk + kh;
-            rg = *src;
-        }
+        for (int u = 0; u < K_PER; ++u) rk[u] = *(const f32x4_t*) (k_p + (size_t) min(t0 + (tid >> 5) + 8 * u, g.B - 1) * QKV);
+        const int t = min(t0 + tid / GR_COLS, g.B - 1);
+        rv.x = v_p[(size_t) t * QKV];
+        rv.y = g.decay[(size_t) t * g.hv + h];
+        rv.z = g.beta[(size_t) t * g.hv + h];
     };
     auto store = [&](int bb) {
 #pragma unroll
-        for (int u = 0; u < QK_PER; ++u) (tid >= 128 ? sk : sq)[bb][u][tid & 127] = rq[u];
-        if (tid < GR_STEPS * GR_COLS) sv[bb][tid / GR_COLS][tid % GR_COLS] = rv;
-        if (tid < 3 * GR_STEPS) ((float*) &sgb[bb][tid & (GR_STEPS - 1)])[tid / GR_STEPS] = rg;
+        for (int u = 0; u < K_PER; ++u) *(f32x4_t*) &sk[bb][(tid >> 5) + 8 * u][k_e] = rk[u];
+        svg[bb][tid / GR_COLS][tid % GR_COLS] = rv;
+    };
+    // q does not go through LDS: a lane keeps its 4 q values of the 32 rows in registers and reloads a
+    // row's right after its use, 32 rows ahead (four waves reading k and q of every row from LDS kept the
+    // LDS busier than the VALU).  Byte offsets stop at the last row.
+    const char* q_b = (const char*) (g.conv_out + (size_t) kh * 128);
+    const uint32_t q_step = (uint32_t) QKV * 4, q_last = (uint32_t) (g.B - 1) * q_step + r8 * 16;
+    uint32_t q_off = r8 * 16;
+    f32x4_t q4[GR_STEPS];
+    auto next_q = [&]() {
+        const f32x4_t v = *(const f32x4_t*) (q_b + q_off);
+        q_off = min(q_off + q_step, q_last);
+        return v;
     };
 
-    // one row of the delta rule from its operands (k . q precomputed):
-    //   kv = dec * (S^T k),  o = dec * (S^T q) + delta * (k.q)  (= (dec S + k delta^T)^T q)
-    float o_row = 0.f;                                      // lane r8 keeps row t0 + r8's output
-    auto row = [&](int st, const float4 k4, const float4 q4, float vv, const float4 gbk) {
-        const float dec = gbk.x, beta = gbk.y, kq = gbk.z;
-        float a = s[0] * k4.x, c = s[0] * q4.x;
-        a = fmaf(s[1], k4.y, a); c = fmaf(s[1], q4.y, c);
-        a = fmaf(s[2], k4.z, a); c = fmaf(s[2], q4.z, c);
-        a = fmaf(s[3], k4.w, a); c = fmaf(s[3], q4.w, c);
-        a = sum32_pl(a);
-        c = sum32_pl(c);
-        const float delta = (vv - dec * a) * beta;
-        const float o = fmaf(dec, c, delta * kq) * 0.08838834764831845f;
-        s[0] = fmaf(k4.x, delta, dec * s[0]);
-        s[1] = fmaf(k4.y, delta, dec * s[1]);
-        s[2] = fmaf(k4.z, delta, dec * s[2]);
-        s[3] = fmaf(k4.w, delta, dec * s[3]);
-        o_row = r8 == st ? o : o_row;
+    float cp[GR_STEPS];                                     // the buffer's rows: this lane's part of S^T q
+    // Row st from its k and gates: kv and the update.  The part of S^T q of the row before (from the
+    // state this row starts with), the decayed state and the loads fill the wait states between the
+    // dependent lane moves; FENCE keeps them there.
+#define FENCE __builtin_amdgcn_sched_barrier(0)
+    auto row = [&](int st, const f32x4_t k4, const f32x4_t qp, const f32x3_t vg, auto&& reads) {
+        float a = s[0] * k4.x, c = s[0] * qp.x;
+        FENCE;
+        a = fmaf(s[1], k4.y, a);
+        c = fmaf(s[1], qp.y, c);
+        FENCE;
+        a = fmaf(s[2], k4.z, a);
+        c = fmaf(s[2], qp.z, c);
+        FENCE;
+        a = fmaf(s[3], k4.w, a);
+        c = fmaf(s[3], qp.w, c);
+        FENCE;
+        const float dec = vg.y;
+        const float m0 = dec * s[0];
+        FENCE;
+        a += dpp_f<DPP_XOR1>(a);
+        FENCE;
+        const float m1 = dec * s[1], m2 = dec * s[2];
+        FENCE;
+        a += dpp_f<DPP_XOR2>(a);
+        FENCE;
+        const float m3 = dec * s[3];
+        reads(0);
+        FENCE;
+        a += dpp_f<DPP_HALF_MIRROR>(a);
+        FENCE;
+        reads(1);
+        FENCE;
+        uint32_t x = __builtin_bit_cast(uint32_t, a + dpp_f<DPP_MIRROR>(a)), y = x;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+        a = __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+        const float delta = (vg.x - dec * a) * vg.z;
+        s[0] = fmaf(k4.x, delta, m0);
+        s[1] = fmaf(k4.y, delta, m1);
+        s[2] = fmaf(k4.z, delta, m2);
+        s[3] = fmaf(k4.w, delta, m3);
+        FENCE;
+        if (st > 0) cp[st - 1] = c;
+    };
+    auto last = [&](const f32x4_t qp) {                     // S^T q after a row
+        float c = s[0] * qp.x;
+        c = fmaf(s[1], qp.y, c);
+        c = fmaf(s[2], qp.z, c);
+        return fmaf(s[3], qp.w, c);
     };
 
-    const int nblk = (g.B + GR_STEPS - 1) / GR_STEPS;
+    const int nfull = g.B / GR_STEPS, rest = g.B - nfull * GR_STEPS;
+#pragma unroll
+    for (int st = 0; st < GR_STEPS; ++st) q4[st] = next_q();
     load(0);
     store(0);
+    // the state has arrived before the loop: without this the wait for it stays inside, behind the
+    // prefetch of the next buffer
+    asm volatile("" : "+v"(s[0]), "+v"(s[1]), "+v"(s[2]), "+v"(s[3]));
     __syncthreads();
-    for (int kb = 0; kb < nblk; ++kb) {
+    // k and gates come from LDS two rows ahead, in register sets used in turn; the loop is unrolled over
+    // the whole buffer, so every LDS address is a constant offset
+    f32x4_t k4[3];
+    f32x3_t vg[3];
+    auto get = [&](int bb, int st) {
+        k4[st % 3] = *(const f32x4_t*) &sk[bb][st][r8 * GR_RPL];
+        vg[st % 3] = *(const f32x3_t*) &svg[bb][st][lc];
+    };
+    float* op = g.o + (size_t) r8 * GV + h * 128 + col;     // lane r8 stores row t0 + r8
+    for (int kb = 0; kb < nfull; ++kb) {
         const int bb = kb & 1, t0 = kb * GR_STEPS;
-        if (kb + 1 < nblk) load(t0 + GR_STEPS);
-        const int n = min(GR_STEPS, g.B - t0);
-        // operands come from LDS one row ahead, alternating between two register sets (rows st and
-        // st + 1), so their latency hides behind the previous row and no copies are needed.  The loop
-        // is unrolled over the whole buffer: every LDS address is a constant offset.
-        float4 kA = *(const float4*) &sk[bb][0][r8 * GR_RPL], qA = *(const float4*) &sq[bb][0][r8 * GR_RPL];
-        float vA = sv[bb][0][lc];
-        float4 pA = sgb[bb][0];
-        float4 kB, qB, pB;
-        float vB;
-        auto pair = [&](int st) {                            // rows st (set A) and st + 1 (set B)
-            const int s1 = min(st + 1, GR_STEPS - 1), s2 = min(st + 2, GR_STEPS - 1);
-            kB = *(const float4*) &sk[bb][s1][r8 * GR_RPL];
-            qB = *(const float4*) &sq[bb][s1][r8 * GR_RPL];
-            vB = sv[bb][s1][lc];
-            pB = sgb[bb][s1];
-            row(st, kA, qA, vA, pA);
-            if (st + 1 >= n) return;                         // workgroup-uniform
-            kA = *(const float4*) &sk[bb][s2][r8 * GR_RPL];
-            qA = *(const float4*) &sq[bb][s2][r8 * GR_RPL];
-            vA = sv[bb][s2][lc];
-            pA = sgb[bb][s2];
-            row(st + 1, kB, qB, vB, pB);
-        };
-        if (n == GR_STEPS) {
+        load(t0 + GR_STEPS);
+        get(bb, 0);
+        get(bb, 1);
 #pragma unroll
-            for (int st = 0; st < GR_STEPS; st += 2) pair(st);
-        } else {
-            for (int st = 0; st < n; st += 2) pair(st);
-        }
+        for (int st = 0; st < GR_STEPS; ++st)
+            row(st, k4[st % 3], q4[st > 0 ? st - 1 : 0], vg[st % 3], [&](int part) {
+                if (part == 0 && st + 2 < GR_STEPS) get(bb, st + 2);
+                if (part == 1 && st > 0) q4[st - 1] = next_q();
+            });
+        cp[GR_STEPS - 1] = last(q4[GR_STEPS - 1]);
+        q4[GR_STEPS - 1] = next_q();
+        const float o = sum32_t(cp) * 0.08838834764831845f;
         // the refill first: it waits for this buffer's loads, long arrived; the output store after it
         // is then waited on by nothing before the next buffer's rows
-        if (kb + 1 < nblk) store(bb ^ 1);
-        if (r8 < n) g.o[(size_t) (t0 + r8) * GV + h * 128 + col] = o_row;
+        store(bb ^ 1);
+        op[(size_t) t0 * GV] = o;
         __syncthreads();
+    }
+    if (rest > 0) {
+        const int bb = nfull & 1;
+#pragma unroll
+        for (int st = 0; st < GR_STEPS; ++st) {
+            cp[st] = 0.f;
+            if (st < rest) {                                 // workgroup-uniform
+                get(bb, st);
+                row(0, k4[st % 3], k4[st % 3], vg[st % 3], [&](int) {});
+                cp[st] = last(q4[st]);
+            }
+        }
+        const float o = sum32_t(cp) * 0.08838834764831845f;
+        if (r8 < rest) op[(size_t) nfull * GR_STEPS * GV] = o;
     }
 #pragma unroll
     for (int i = 0; i < GR_RPL; ++i) S[(size_t) (r8 * GR_RPL + i) * 128 + col] = s[i];
 }
+#undef FENCE
 
 // y = bf16(o * rsqrt(mean o^2 + eps) * gamma * sigmoid(z)) per (head, row); grid (hv, B), 128 threads
 // (pf_gdn_rmsnorm_gate_parallel, src/wzy_qsa_wmma.cuh:176-195)
@@ -1157,7 +1208,6 @@ int launch_pf_gdn(const PfGdn& g, hipStream_t st) {
     hipLaunchKernelGGL(pf_gdn_ab_kernel, dim3((g.B * g.hv + 255) / 256), dim3(256), 0, st, g);
     hipLaunchKernelGGL(pf_gdn_conv_kernel, dim3(QKV / 128, (g.B + CV_ROWS - 1) / CV_ROWS), dim3(128), 0, st, g);
     hipLaunchKernelGGL(pf_gdn_hist_kernel, dim3((QKV + 255) / 256), dim3(256), 0, st, g);
-    hipLaunchKernelGGL(pf_gdn_kq_kernel, dim3((g.B * g.hk + 7) / 8), dim3(256), 0, st, g);
     hipLaunchKernelGGL(pf_gdn_recur_kernel, dim3(g.hv * 128 / GR_COLS), dim3(256), 0, st, g);
     hipLaunchKernelGGL(pf_gdn_norm_kernel, dim3(g.hv, g.B), dim3(128), 0, st, g);
     WZY_LAUNCH_CHECK();
