@@ -362,10 +362,13 @@ def test_stage_prefill_matches_oracle(wz, orc, gpu, p0, B, prefix):
         st.close()
 
 
-@pytest.mark.parametrize("p0,B,prefix", [(0, 31, 0), (0, 32, 0), (0, 33, 0), (3, 64, 3), (0, 97, 0)])
+@pytest.mark.parametrize("p0,B,prefix", [(0, 31, 0), (0, 32, 0), (0, 33, 0), (3, 64, 3), (0, 129, 0)])
 def test_stage_prefill_at_recurrence_buffer_edges(wz, orc, gpu, p0, B, prefix):
     """Chunks around multiples of the 32 rows the delta rule keeps in flight: no full buffer, full
-    buffers only, and both with a rest of one row."""
+    buffers only, and both with a rest of one row.  (129 rows rather than 97: the comparison leaves out
+    rows within 1e-4 of a routing tie and wants 99 % of them left; of the 388 layer-rows of the 97 tokens
+    drawn for that length 3 or 4 lie at that distance, depending on the rounding of the layers before.)
+    """
     test_stage_prefill_matches_oracle(wz, orc, gpu, p0, B, prefix)
 
 

@@ -16,10 +16,12 @@
 //  QSA           pf_qsa_prep (q / k / indexer-q norms + RoPE, INT8 KV append), pf_idx_append (the
 //                indexer keys of every block the chunk completes, one workgroup per block, then
 //                pf_idx_tail), block scores on fp16 MFMA (pf_score), top-k with the decode kernel,
-//                pf_attn (sparse GQA attention on fp16 MFMA, 64 cells per load step, a 32-cell
-//                online softmax).
+//                pf_attn (sparse GQA attention on fp16 MFMA, K and V from memory straight into the
+//                matrix operands).
 // reference: PrefillStageCtx::run_stage_prefill and its kernels (src/wzy_prefill_tc.cuh:20-98,
 // 546-1058; src/wzy_qsa_wmma.cuh:5-489), with cuBLAS fp16 GEMMs replaced by bf16 MFMA GEMMs.
+#include <type_traits>
+
 #include "wzy_device.h"
 #include "wzy_host.h"
 #include "wzy_prefill.h"
@@ -30,9 +32,10 @@ using namespace wzy;
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x3_t __attribute__((ext_vector_type(3)));
+typedef int i32x2_t __attribute__((ext_vector_type(2)));
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
 namespace {
 
@@ -859,236 +862,230 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
 }
 
 // Sparse GQA attention of one row and one KV head (grid (kvh, B), 256 threads): the group's query
-// heads (up to 16, rows of a 16 x 16 fp16 MFMA tile) against the selected cells, 64 per load step.
-// Per step: K of 64 cells dequantised to fp16 in LDS (row major), scores on
-// v_mfma_f32_16x16x16_f16 (wave w: cells 16w .. 16w+15, all 256 dims as two 128-dim chains added in
-// fp32), then two 32-cell softmax blocks in order (the online softmax per head with fp16 weights,
-// as the reference's 32-cell steps), V dequantised into LDS transposed (dims x cells) and P.V on
-// MFMA into the accumulators, rescaled by exp(m_old - m_new) before each block.  The next step's K
-// and V codes (32 KB) are loaded while a step computes, from cell ids staged in LDS a step earlier.  out = acc / max(l, 1e-20) * sigmoid(gate),
-// bf16.
-constexpr int AT_C = 64;                      // cells per load step (two softmax blocks of 32)
-constexpr int AT_B = 32;                      // cells per softmax block
-constexpr int AT_QLD = 256 + 8;               // LDS row strides (halves)
-constexpr int AT_VLD = AT_C + 4;
+// heads (up to 16, columns of a 16 x 16 fp16 MFMA tile) against the selected cells.  Each wave takes
+// every fourth 32-cell chunk through a softmax of its own; the four are merged at the end.
+//
+// Nothing of the loop goes through LDS but the chunk's cell ids.  K and V codes are loaded straight into
+// the lanes that feed them to the matrix cores, 16 bytes at a time, and dequantised there:
+//   S^T = K Q^T   A = K: lane l holds cell l % 16, its 16-byte pieces at dims 64 u + 16 (l / 16); the sum
+//                 over dims may run in any order, so Q^T (B, in registers) takes the same dims.
+//   O^T = V^T P^T the accumulator layout of S^T (cells 4 (l / 16) + i of head l % 16) is the B layout of
+//                 P^T, so the weights never leave their lane; A = V^T: lane l holds dims 16 (l % 16) + t of
+//                 the same eight cells, regrouped from cells x dims to dims x cells by byte permutes.
+// Codes become fp16 exactly as 1024 + (code + 128) - 1152 (a byte under the exponent of 1024), then
+// code * scale is rounded to fp16 once, two at a time, as a product of fp16 numbers.
+// The softmax keeps a reference exponent per head that a chunk's maximum moves only when it exceeds it by
+// more than 2^AT_LAZY (fp16 weights up to 64 lose nothing), so most chunks rescale no accumulator.
+// K of the next chunk is loaded once this chunk's codes are converted, V likewise.  out = acc / max(l,
+// 1e-20) * sigmoid(gate), bf16.
+// What bounds it: the gather (528 bytes per cell, row and KV head, from the Infinity Cache where a context
+// exceeds the L2) and about 480 VALU operations per 32 cells and wave for the conversions.  Against the
+// kernel before it, which staged K and a transposed V through LDS with three barriers per 64 cells: 8,192
+// rows over 2,048 of 33-41 thousand cells 3,400 -> 1,775 us (9.8 TB/s gathered), 1,301 rows over 2,048 of 9-10
+// thousand 530 -> 301 us.
+constexpr int AT_C = 32;                      // cells per wave and step
+constexpr float AT_LAZY = 6.0f;               // log2 units
+constexpr int AT_OLD = 256 + 4;               // LDS row stride of the partial outputs (floats)
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
-// LDS placement of K dim d in a cell row: the upper 128 dims swap neighbouring 4-dim groups, so the
-// 64 lanes of a K staging store (16 cells x 4 dim quarters; quarters q and q + 2 lie 64 words apart)
-// spread over more banks.  The score reads take one 16-dim slice, so their pattern is unchanged.
-// This swap, the V^T rotation below and the pitches of V^T and sS were chosen by measuring LDS bank
-// conflict counts and the prefill time of variants.
-WZY_DEV int at_kcol(int d) { return d ^ ((d >> 5) & 4); }
-// LDS column of cell c in row d of V^T: the cells are rotated by 8 * ((d / 16) % 8) (mod 64), so the
-// 16 lanes that stage one cell group (rows 16 apart, which the pitch alone would put in one bank
-// group) start in different banks; the 16 rows a P.V read spans share one rotation.
-WZY_DEV int at_vcol(int d, int c) { return (c + 8 * ((d >> 4) & 7)) & (AT_C - 1); }
+// bytes x0, x1 / x2, x3 of the biased codes w -> 1024 + x, minus 1152: the codes as fp16 pairs
+WZY_DEV f16x2_t at_lo(uint32_t w) {
+    return __builtin_bit_cast(f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) - (_Float16) 1152.0f;
+}
+WZY_DEV f16x2_t at_hi(uint32_t w) {
+    return __builtin_bit_cast(f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u)) - (_Float16) 1152.0f;
+}
+WZY_DEV f16x8_t at_join(f16x2_t a, f16x2_t b, f16x2_t c, f16x2_t d) {
+    return f16x8_t{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+// eight K codes times their scale
+WZY_DEV f16x8_t at_k8(uint32_t a, uint32_t b, f16x2_t sc) {
+    a ^= 0x80808080u;
+    b ^= 0x80808080u;
+    return at_join(at_lo(a) * sc, at_hi(a) * sc, at_lo(b) * sc, at_hi(b) * sc);
+}
+// maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (inline assembly as in sum32_pl)
+template <bool MAX>
+WZY_DEV float at_rows(float v) {
+    uint32_t x = __builtin_bit_cast(uint32_t, v), y = x;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+    const float a = __builtin_bit_cast(float, x), b = __builtin_bit_cast(float, y);
+    const float r = MAX ? fmaxf(a, b) : a + b;
+    x = y = __builtin_bit_cast(uint32_t, r);
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+    const float c = __builtin_bit_cast(float, x), d = __builtin_bit_cast(float, y);
+    return MAX ? fmaxf(c, d) : c + d;
+}
 
-WZY_DEV f16x4_t h4_from(const _Float16* p) { return *(const f16x4_t*) p; }
-
-__global__ void __launch_bounds__(256, 3) pf_attn_kernel(PfAttn a) {
-    // K of a step and then its V^T share one region (37 KB instead of 70), so three workgroups fit a
-    // CU: the scores read K, V is staged after every wave is done with K, P.V reads V^T.
-    __shared__ __align__(16) _Float16 sU[256 * AT_VLD];
-    _Float16 (*const sK)[AT_QLD] = (_Float16 (*)[AT_QLD]) sU;
-    _Float16 (*const sVt)[AT_VLD] = (_Float16 (*)[AT_VLD]) sU;
-    static_assert(AT_C * AT_QLD <= 256 * AT_VLD, "K fits the shared region");
-    __shared__ __align__(16) _Float16 sP[2][16][AT_B + 8];
-    __shared__ float sS[16][AT_C + 4];                 // pitch 68: a wave's score writes (rows 4 apart) hit distinct banks
-    __shared__ float s_m[16], s_l[16], s_al[2][16];
-    __shared__ int sIds[2][AT_C];                 // selected cell ids of the next two steps
+// O32: byte offsets into the code planes fit 32 bits (launch_pf_attn), so a cell's address is the plane's
+// base and one register, kept in LDS ready made.
+template <bool O32>
+__global__ void __launch_bounds__(256, 2) pf_attn_kernel(PfAttn a) {
+    typedef typename std::conditional<O32, uint32_t, uint64_t>::type off_t;
+    __shared__ __align__(16) float sO[4][16][AT_OLD];
+    __shared__ __align__(16) off_t sOff[4][2][AT_C];     // per wave: code offsets of this chunk's cells and the next's
+    __shared__ float s_m[4][16], s_l[4][16];
     const QsaDims& dm = a.dm;
-    const int j = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int hd = 256, kvd = dm.kvh * hd, gq = dm.qh / dm.kvh, scg = hd / 64;
+    const int j = blockIdx.x, t = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hd = 256, kvd = dm.kvh * hd, gq = dm.qh / dm.kvh;
     const int n_kv = *a.pos + t + 1;
     const int width = min(n_kv, dm.topk);
     const int* ids = a.sel + (size_t) t * dm.topk;
     const float* qg = a.qg + (size_t) t * dm.qh * 2 * hd;
+    const int l16 = lane & 15, g = lane >> 4;
 
-    const int l16 = lane & 15, kq4 = lane >> 4;   // MFMA 16x16x16: row/col l16, k quad kq4
-    // the A operand of every score MFMA, held in registers: q[head l16][16 kk + 4 kq4 .. +3] / 16
-    f16x4_t qa[16];
+    // Q^T: q[head l16][64 u + 16 g + 8 half .. +7] / 16 for every (u, half)
+    f16x8_t qb[8];
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-        const float4 q4 = l16 < gq ? *(const float4*) (qg + (size_t) (j * gq + l16) * 2 * hd + kk * 16 + 4 * kq4)
-                                   : make_float4(0.f, 0.f, 0.f, 0.f);
-        qa[kk] = f16x4_t{(_Float16) (q4.x * 0.0625f), (_Float16) (q4.y * 0.0625f), (_Float16) (q4.z * 0.0625f),
-                         (_Float16) (q4.w * 0.0625f)};
+    for (int uh = 0; uh < 8; ++uh) {
+        const float* qp = qg + (size_t) (j * gq + min(l16, gq - 1)) * 2 * hd + 64 * (uh >> 1) + 16 * g + 8 * (uh & 1);
+        const f32x4_t x = *(const f32x4_t*) qp, y = *(const f32x4_t*) (qp + 4);
+        const float z = l16 < gq ? 0.0625f : 0.f;
+        qb[uh] = f16x8_t{(_Float16) (x.x * z), (_Float16) (x.y * z), (_Float16) (x.z * z), (_Float16) (x.w * z),
+                         (_Float16) (y.x * z), (_Float16) (y.y * z), (_Float16) (y.z * z), (_Float16) (y.w * z)};
     }
-    if (tid < 16) {
-        s_m[tid] = -1e30f;
-        s_l[tid] = 0.f;
-    }
-    // K staging: thread -> cell kc = tid / 4, dims 64 * (tid % 4) .. +63 (64 code bytes, one scale)
-    const int kc = tid >> 2, kd0 = (tid & 3) * 64;
-    // V staging: thread -> cells 4 * (tid / 16) .. +3, dims 16 * (tid % 16) .. +15
-    const int vc0 = (tid >> 4) * 4, vd0 = (tid & 15) * 16;
-    uint4 kq[4], vq[4];
-    uint16_t ksc = 0, vsc[4];
-    int rid = 0;
-    // the ids of a step are read from global memory two steps ahead and staged in LDS, so the K / V
-    // loads of the next step depend on no global load of their own step
-    auto load_ids = [&](int base) { rid = ids[base + min(tid & (AT_C - 1), width - base - 1)]; };
-    auto store_ids = [&](int slot) {
-        if (tid < AT_C) sIds[slot][tid] = rid;
-    };
-    auto load_k = [&](int base, int slot) {
-        const int cnt = min(AT_C, width - base);
-        {
-            const bool ok = kc < cnt;
-            const size_t p = qsa_kv_slot(sIds[slot][ok ? kc : 0], dm);
-            const int8_t* kp = a.kv.kq + p * kvd + (size_t) j * hd + kd0;
+    f32x4_t acc[16];                              // O^T: dims 16 (4 g + i) + t of head l16
 #pragma unroll
-            for (int u = 0; u < 4; ++u) kq[u] = ok ? *(const uint4*) (kp + 16 * u) : make_uint4(0, 0, 0, 0);
-            ksc = ok ? a.kv.ks[p * (kvd / 64) + (size_t) j * scg + kd0 / 64] : (uint16_t) 0;
-        }
+    for (int i = 0; i < 16; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m_ref = -1e30f, l_sum = 0.f;            // per head l16; l_sum is this lane's part
+
+    const int nch = (width + AT_C - 1) / AT_C;    // chunks; this wave takes w, w + 4, ...
+    // a cell's codes start at its offset, its scales (fp16 per 64 codes) at a 32nd of it
+    const char* kb = (const char*) (a.kv.kq + (size_t) j * hd);
+    const char* vb = (const char*) (a.kv.vq + (size_t) j * hd);
+    const char* ksb = (const char*) (a.kv.ks + (size_t) j * 4);
+    const char* vsb = (const char*) (a.kv.vs + (size_t) j * 4);
+    const off_t ko = 16 * g, vo = 16 * l16, vso = 2 * (l16 >> 2);
+    // cells past the selection repeat its last one: every load is unconditional
+    auto read_id = [&](int c) {
+        return (off_t) qsa_kv_slot(ids[max(0, min(AT_C * c + (lane & 31), width - 1))], dm) * (off_t) kvd;
     };
-    auto load_v = [&](int base, int slot) {
-        const int cnt = min(AT_C, width - base);
+
+    i32x4_t kr[2][4];                             // K codes of cells l16, 16 + l16: pieces u = 0 .. 3
+    i32x2_t ksr[2];                               // and their four scales
+    i32x4_t vr[8];                                // V codes of cells 4 g + i, 16 + 4 g + i
+    uint16_t vsr[8];
+#define AT_LOAD_K(slot)                                                                        \
+    _Pragma("unroll") for (int c_ = 0; c_ < 2; ++c_) {                                         \
+        const off_t p_ = sOff[w][slot][16 * c_ + l16];                                         \
+        _Pragma("unroll") for (int u_ = 0; u_ < 4; ++u_)                                       \
+            kr[c_][u_] = *(const i32x4_t*) (kb + (off_t) (p_ + ko) + 64 * u_);                 \
+        ksr[c_] = *(const i32x2_t*) (ksb + (off_t) (p_ >> 5));                                 \
+    }
+#define AT_LOAD_V(slot)                                                                        \
+    _Pragma("unroll") for (int c_ = 0; c_ < 8; ++c_) {                                         \
+        const off_t p_ = sOff[w][slot][16 * (c_ >> 2) + 4 * g + (c_ & 3)];                     \
+        vr[c_] = *(const i32x4_t*) (vb + (off_t) (p_ + vo));                                   \
+        vsr[c_] = *(const uint16_t*) (vsb + (off_t) ((p_ >> 5) + vso));                        \
+    }
+    off_t rid = 0;
+    if (w < nch) {
+        rid = read_id(w);
+        if (lane < AT_C) sOff[w][0][lane] = rid;
+        rid = read_id(w + 4);
+        AT_LOAD_K(0)
+        AT_LOAD_V(0)
+    }
+    for (int c = w, it = 0; c < nch; c += 4, ++it) {
+        const int nx = (it + 1) & 1;
+        if (lane < AT_C) sOff[w][nx][lane] = rid;
+        rid = read_id(c + 8);
+        // S^T of the chunk's two 16-cell tiles
+        f32x4_t sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const bool ok = vc0 + u < cnt;
-            const size_t p = qsa_kv_slot(sIds[slot][ok ? vc0 + u : 0], dm);
-            vq[u] = ok ? *(const uint4*) (a.kv.vq + p * kvd + (size_t) j * hd + vd0) : make_uint4(0, 0, 0, 0);
-            vsc[u] = ok ? a.kv.vs[p * (kvd / 64) + (size_t) j * scg + vd0 / 64] : (uint16_t) 0;
-        }
-    };
-    auto store_k = [&]() {
-        const _Float16 s = __builtin_bit_cast(_Float16, ksc);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint32_t wv[4] = {kq[u].x, kq[u].y, kq[u].z, kq[u].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                f16x4_t v;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) v[b] = (_Float16) (int8_t) (wv[i] >> (8 * b)) * s;
-                *(f16x4_t*) &sK[kc][at_kcol(kd0 + 16 * u + 4 * i)] = v;
+            for (int ct = 0; ct < 2; ++ct) {
+                const uint32_t sw = (uint32_t) (u < 2 ? ksr[ct].x : ksr[ct].y);
+                const uint32_t s2 = __builtin_amdgcn_perm(sw, sw, (u & 1) ? 0x03020302u : 0x01000100u);
+                const f16x2_t s = __builtin_bit_cast(f16x2_t, s2);
+                const f16x8_t k0 = at_k8((uint32_t) kr[ct][u].x, (uint32_t) kr[ct][u].y, s);
+                const f16x8_t k1 = at_k8((uint32_t) kr[ct][u].z, (uint32_t) kr[ct][u].w, s);
+                sc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qb[2 * u], sc[ct], 0, 0, 0);
+                sc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qb[2 * u + 1], sc[ct], 0, 0, 0);
             }
         }
-    };
-    auto store_v = [&]() {
-        _Float16 vs[4];
+        AT_LOAD_K(nx)
+        // softmax weights of this lane's eight cells of head l16, in units of 2^m_ref
+        const int left = width - AT_C * c - 4 * g;        // cell (ct, i) is selected iff 16 ct + i < left
+        float z[8], mx = -1e30f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) vs[u] = __builtin_bit_cast(_Float16, vsc[u]);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {               // dim vd0 + i of the 4 cells
-            f16x4_t v;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t word = i < 4 ? vq[u].x : i < 8 ? vq[u].y : i < 12 ? vq[u].z : vq[u].w;
-                v[u] = (_Float16) (int8_t) (word >> (8 * (i & 3))) * vs[u];
-            }
-            *(f16x4_t*) &sVt[vd0 + i][at_vcol(vd0, vc0)] = v;
+        for (int e = 0; e < 8; ++e) {
+            z[e] = sc[e >> 2][e & 3] * 1.44269504f;
+            if (16 * (e >> 2) + (e & 3) < left) mx = fmaxf(mx, z[e]);
         }
-    };
-
-    f32x4_t acc[4];                               // out[h = 4*(lane/16) + i][d = 64w + 16db + lane%16]
+        mx = at_rows<true>(mx);
+        if (__any(mx > m_ref + AT_LAZY)) {
+            const float m_new = fmaxf(m_ref, mx), al = __builtin_amdgcn_exp2f(m_ref - m_new);
+            m_ref = m_new;
+            l_sum *= al;
 #pragma unroll
-    for (int db = 0; db < 4; ++db) acc[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    if (width > 0) {
-        load_ids(0);
-        store_ids(0);
+            for (int i = 0; i < 16; ++i) acc[i] *= al;
+        }
+        f16x8_t pw;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float p = 16 * (e >> 2) + (e & 3) < left ? __builtin_amdgcn_exp2f(z[e] - m_ref) : 0.f;
+            l_sum += p;
+            pw[e] = (_Float16) p;
+        }
+        // O^T: the eight cells of four dims at a time
+        f16x2_t vs2[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            vs2[q] = f16x2_t{__builtin_bit_cast(_Float16, vsr[2 * q]), __builtin_bit_cast(_Float16, vsr[2 * q + 1])};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t d01[4], d23[4];                      // per cell pair: bytes of dims 4i, 4i+1 / 4i+2, 4i+3
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t x = (uint32_t) vr[2 * q][i] ^ 0x80808080u, y = (uint32_t) vr[2 * q + 1][i] ^ 0x80808080u;
+                d01[q] = __builtin_amdgcn_perm(y, x, 0x05010400u);
+                d23[q] = __builtin_amdgcn_perm(y, x, 0x07030602u);
+            }
+            acc[4 * i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                at_join(at_lo(d01[0]) * vs2[0], at_lo(d01[1]) * vs2[1], at_lo(d01[2]) * vs2[2], at_lo(d01[3]) * vs2[3]), pw,
+                acc[4 * i], 0, 0, 0);
+            acc[4 * i + 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                at_join(at_hi(d01[0]) * vs2[0], at_hi(d01[1]) * vs2[1], at_hi(d01[2]) * vs2[2], at_hi(d01[3]) * vs2[3]), pw,
+                acc[4 * i + 1], 0, 0, 0);
+            acc[4 * i + 2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                at_join(at_lo(d23[0]) * vs2[0], at_lo(d23[1]) * vs2[1], at_lo(d23[2]) * vs2[2], at_lo(d23[3]) * vs2[3]), pw,
+                acc[4 * i + 2], 0, 0, 0);
+            acc[4 * i + 3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                at_join(at_hi(d23[0]) * vs2[0], at_hi(d23[1]) * vs2[1], at_hi(d23[2]) * vs2[2], at_hi(d23[3]) * vs2[3]), pw,
+                acc[4 * i + 3], 0, 0, 0);
+        }
+        AT_LOAD_V(nx)
     }
+#undef AT_LOAD_K
+#undef AT_LOAD_V
+    // merge the waves: out[d] = sum_w 2^(m_w - m) acc_w[d] / sum_w 2^(m_w - m) l_w
+    l_sum = at_rows<false>(l_sum);
+    if (g == 0) {
+        s_m[w][l16] = m_ref;
+        s_l[w][l16] = l_sum;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            *(f32x4_t*) &sO[w][l16][16 * (4 * g + i) + 4 * q] =
+                f32x4_t{acc[4 * q][i], acc[4 * q + 1][i], acc[4 * q + 2][i], acc[4 * q + 3][i]};
     __syncthreads();
-    if (width > 0) {
-        load_k(0, 0);
-        load_v(0, 0);
-    }
-    if (AT_C < width) load_ids(AT_C);
-    if (width > 0) store_k();
-    if (AT_C < width) store_ids(1);
-    __syncthreads();
-    // per step: the next step's K loads go out first; V of this step (in registers since the middle
-    // of the previous step) is staged once the scores are done, and the next step's V loads follow
-    for (int base = 0, stp = 0; base < width; base += AT_C, ++stp) {
-        const int cnt = min(AT_C, width - base);
-        const bool more = base + AT_C < width, more2 = base + 2 * AT_C < width;
-        if (more) load_k(base + AT_C, (stp + 1) & 1);
-        if (more2) load_ids(base + 2 * AT_C);
-        // scores: wave w -> cells 16w .. 16w+15, dims 0-127 and 128-255 as separate chains
-        if (16 * w < cnt) {
-            f32x4_t sc0 = {0.f, 0.f, 0.f, 0.f}, sc1 = {0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < gq; ++h) {                        // thread = dim
+        const float m = fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h]));
+        float o = 0.f, l = 0.f;
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                sc0 = __builtin_amdgcn_mfma_f32_16x16x16f16(qa[kk], h4_from(&sK[16 * w + l16][kk * 16 + 4 * kq4]), sc0,
-                                                            0, 0, 0);
-                sc1 = __builtin_amdgcn_mfma_f32_16x16x16f16(qa[8 + kk], h4_from(&sK[16 * w + l16][at_kcol(128 + kk * 16 + 4 * kq4)]),
-                                                            sc1, 0, 0, 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sS[4 * kq4 + i][16 * w + l16] = sc0[i] + sc1[i];
+        for (int v = 0; v < 4; ++v) {
+            const float f = __builtin_amdgcn_exp2f(s_m[v][h] - m);
+            l = fmaf(s_l[v][h], f, l);
+            o = fmaf(sO[v][h][tid], f, o);
         }
-        __syncthreads();
-        store_v();                                   // K is no longer read: V^T takes the region
-        if (more) load_v(base + AT_C, (stp + 1) & 1);
-        // online softmax, two 32-cell blocks in order: wave w -> heads 4w .. 4w+3, two per pass
-        // (lane halves), lane = cell of the block
-#pragma unroll
-        for (int pass = 0; pass < 2; ++pass) {
-            const int h = 4 * w + 2 * pass + (lane >> 5), c = lane & 31;
-            float m_run = h < gq ? s_m[h] : 0.f, l_run = h < gq ? s_l[h] : 0.f;
-#pragma unroll
-            for (int sb = 0; sb < 2; ++sb) {
-                const int cc = AT_B * sb + c;
-                const bool ok = cc < cnt && h < gq;
-                const float sv = ok ? sS[h][cc] : -1e30f;
-                const float rmax = max32(sv);
-                const float m_new = fmaxf(m_run, rmax);
-                const float al = h < gq ? __expf(m_run - m_new) : 1.f;
-                const float pw = ok ? __expf(sv - m_new) : 0.f;
-                const float psum = sum32(pw);
-                sP[sb][h][c] = (_Float16) pw;
-                l_run = l_run * al + psum;
-                m_run = m_new;
-                if (c == 0) s_al[sb][h] = al;
-            }
-            if (c == 0 && h < gq) {
-                s_m[h] = m_run;
-                s_l[h] = l_run;
-            }
-        }
-        __syncthreads();
-        // P.V: wave w -> dims 64w .. 64w+63 (four 16-dim blocks), per softmax block two k16 slices
-#pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-            if (AT_B * sb >= cnt) break;             // workgroup-uniform
-            float al[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) al[i] = s_al[sb][4 * kq4 + i];
-#pragma unroll
-            for (int db = 0; db < 4; ++db)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[db][i] *= al[i];
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const f16x4_t pv = h4_from(&sP[sb][l16][ks * 16 + 4 * kq4]);
-#pragma unroll
-                for (int db = 0; db < 4; ++db) {
-                    const int d = 64 * w + 16 * db + l16;
-                    const f16x4_t vv = h4_from(&sVt[d][at_vcol(d, AT_B * sb + ks * 16 + 4 * kq4)]);
-                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x16f16(pv, vv, acc[db], 0, 0, 0);
-                }
-            }
-        }
-        __syncthreads();
-        if (more) store_k();
-        if (more2) store_ids(stp & 1);
-        __syncthreads();
-    }
-    // acc[db][i] = O[head 4*kq4 + i][dim 64w + 16db + l16]
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int h = 4 * kq4 + i;
-        if (h >= gq) continue;
-        const float inv = 1.0f / fmaxf(s_l[h], 1e-20f);
-#pragma unroll
-        for (int db = 0; db < 4; ++db) {
-            const int d = 64 * w + 16 * db + l16;
-            const float gate = qg[(size_t) (j * gq + h) * 2 * hd + hd + d];
-            const float v = (acc[db][i] * inv) / (1.0f + __expf(-gate));
-            a.out[(size_t) t * dm.qh * hd + (size_t) (j * gq + h) * hd + d] = f_to_bf16(v);
-        }
+        const float gate = qg[(size_t) (j * gq + h) * 2 * hd + hd + tid];
+        const float y = (o * (1.0f / fmaxf(l, 1e-20f))) / (1.0f + __expf(-gate));
+        a.out[(size_t) t * dm.qh * hd + (size_t) (j * gq + h) * hd + tid] = f_to_bf16(y);
     }
 }
 
@@ -1253,7 +1250,10 @@ int launch_pf_attn(const PfAttn& a, int B, hipStream_t st) {
     WZY_TRY(qsa_check_dims(a.dm));
     WZY_REQUIRE(a.dm.hd == 256 && a.dm.qh / a.dm.kvh <= 16 && a.dm.window == 0, "pf_attn: head layout unsupported");
     WZY_REQUIRE(B >= 1 && B <= 65535, "pf_attn: %d rows", B);
-    hipLaunchKernelGGL(pf_attn_kernel, dim3(a.dm.kvh, B), dim3(256), 0, st, a);
+    if ((uint64_t) a.dm.ctx_max * a.dm.kvh * a.dm.hd <= UINT32_MAX)
+        hipLaunchKernelGGL(pf_attn_kernel<true>, dim3(a.dm.kvh, B), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(pf_attn_kernel<false>, dim3(a.dm.kvh, B), dim3(256), 0, st, a);
     WZY_LAUNCH_CHECK();
     return WZY_OK;
 }
