@@ -146,7 +146,7 @@ size_t wzy_moe_prefill_workspace_bytes(int n_embd, int n_ff, int n_exp, int top_
 
 /* MoE block for a prefill chunk of n_tok rows of x [n_tok x n_embd] (fp32), on MFMA:
  * x rounded to bf16 -> router logits (bf16 GEMM) -> softmax top-k per token (the decode rule) ->
- * entries grouped by expert into tiles of up to 256 -> routed gate|up (NVFP4 dequantised to bf16
+ * entries grouped by expert into tiles of up to 128 -> routed gate|up (NVFP4 dequantised to bf16
  * MFMA operands; the fp32 tensor scale applied to the accumulators) + SwiGLU (bf16) -> down, fp32
  * per entry -> comb = sigmoid(sgate.x) * shared(x) + sum_k w_k * expert_k(x), summed per token in
  * slot order (results do not depend on the order entries reach their expert); the shared expert's
@@ -164,6 +164,8 @@ int wzy_moe_prefill(const wzy_moe_weights* w, const float* x, int n_tok, float* 
  * its launch groups on `stream`; us_stages[8] = mean microseconds of
  *   0 x -> bf16, 1 router GEMM, 2 routing + shared gate, 3 expert tiles and entry lists,
  *   4 shared gate|up, 5 shared down, 6 routed gate|up, 7 routed down + per-token combine.
+ * Chunks below 8,192 tokens run the shared expert inside the routed launches: groups 4 and 5 are then
+ * empty and 6 and 7 include it.
  * Counterpart of the reference's WZY_PF_PROF phase timers (src/wzy_prefill_tc.cuh:734-741). */
 int wzy_moe_prefill_time(const wzy_moe_weights* w, const float* x, int n_tok, float* comb, void* workspace,
                          size_t workspace_bytes, int iters, float* us_stages, void* stream);

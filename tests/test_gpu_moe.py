@@ -498,6 +498,24 @@ def test_moe_prefill_config1_shape(wz, orc, gpu):
     assert err < 3e-3, err
 
 
+def test_moe_prefill_tile_sizes_agree(wz, gpu):
+    """The block picks 64- or 128-entry expert tiles by the entries per expert (60 of 64 experts top-8 at 480
+    tokens), and an expert past a tile's size is cut into equal ones; an entry's sums depend on neither: the
+    same tokens in a longer chunk give the same rows, bit for bit.  n_ff 640 leaves the down projection an
+    odd number of weight chunks, 400 / 480 / 481 / 1,200 tokens end row blocks of every kind."""
+    print("case moe_prefill_tile_sizes", flush=True)
+    D, F, E, K, N = 512, 640, 64, 8, 1200
+    m = mi.make_layer(wz, 9, 0, D, F, E, K)
+    x = mi.make_x(wz, 9, 0, N, D)
+    w, keep = device_layer(wz, m)
+    comb, ids, wts = run_gpu_prefill(wz, w, x, N)
+    for n in (1, 33, 65, 400, 480, 481):
+        c, i, v = run_gpu_prefill(wz, w, x[:n], n)
+        np.testing.assert_array_equal(i, ids[:n * K])
+        np.testing.assert_array_equal(v, wts[:n * K])
+        np.testing.assert_array_equal(c, comb[:n * D])
+
+
 def test_moe_prefill_rejects_bad_shapes(wz, gpu):
     D, F, E, K = 256, 128, 48, 4                  # 48 experts: not a multiple of 64
     m = mi.make_layer(wz, 1, 0, D, F, 64, K, blobs=[])

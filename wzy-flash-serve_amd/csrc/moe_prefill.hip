@@ -5,19 +5,22 @@
 //   2. pf_gemm     router logits [N x E] = x . router^T                      (bf16 weights)
 //   3. pf_route    per token, one wave: softmax top-K (the decode routing: probability desc, id asc,
 //                  weights renormalised by max(sum, 2^-14)) and the shared-expert gate sg = sgate . x
-//   4. pf_hist, pf_tiles, pf_scatter: entries (token, slot) grouped by expert into tiles of up to
-//                  256 (LDS-histogram ranks, one reserving atomic per expert and workgroup, one scan)
-//   5. pf_expert<gate|up, Q8_0>  shared expert, dense 128-token blocks, SwiGLU -> sh_act bf16 [N x F]
-//   6. pf_expert<down, Q8_0>     shared expert, dense 256-token blocks -> comb = sigmoid(sg) * shared
+//   4. pf_hist, pf_tiles, pf_scatter: entries (token, slot) grouped by expert into tiles of up to 64 or
+//                  128 (LDS-histogram ranks, one reserving atomic per expert and workgroup, one scan)
+//   5. pf_expert<gate|up, Q8_0>  shared expert, dense token blocks, SwiGLU -> sh_act bf16 [N x F]
+//   6. pf_expert<down, Q8_0>     shared expert, dense token blocks -> comb = sigmoid(sg) * shared
 //   7. pf_expert<gate|up, NVFP4> routed, one expert tile per workgroup, SwiGLU -> act bf16 [N*K x F]
 //   8. pf_expert<down, NVFP4>    routed -> y fp32 [N*K x D] per entry; pf_combine: comb[t] +=
 //                  sum_k w_k * y[pos(t, k)] in slot order (no float atomics)
-// pf_expert: 8 waves, 256 weight rows per workgroup, up to 256 A rows; weights staged through LDS in
-// coalesced 128-k chunks and dequantised by each lane into its v_mfma_f32_32x32x16_bf16 B fragment
+// Shorter chunks run 5 in the launch of 7 and 6 in the launch of 8.
+// pf_expert: 8 waves, 256 weight rows per workgroup, up to 128 A rows; weights staged through LDS in
+// coalesced 64-byte pieces of a row and dequantised by each lane into its v_mfma_f32_32x32x16_bf16 B fragment
 // (e2m1 x e4m3 block scale is exact in bf16, the fp32 tensor scale goes onto the accumulators;
 // Q8_0 code x fp16 scale is rounded to bf16).  pf_gemm: 64 x 64 LDS-tiled bf16 GEMM (router).
 // reference: pf_moe_gu_wmma_kernel, pf_moe_down_wmma_kernel, the tile builder and the shared/router
 // prefill GEMMs (src/wzy_prefill_tc.cuh:99-443), with fp16 replaced by bf16.
+#include <type_traits>
+
 #include "wzy_device.h"
 #include "wzy_host.h"
 #include "wzy_moe.h"
@@ -29,18 +32,19 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 namespace {
 
 constexpr int PB = 64;             // router GEMM: tile rows (M), weight rows (N) and K step
 constexpr int PB_LD = PB + 8;      // LDS row stride in bf16 (16-byte aligned rows, staggered banks)
 constexpr int PF_MAX_E = 1024;
-constexpr int MT = 256;            // expert GEMM: entries per tile (8 MFMA row blocks of 32)
 constexpr int EK = 64;             // expert GEMM: K step between barriers (four MFMA k16 slices)
 constexpr int EA_LD = EK + 8;      // LDS row stride of the staged activations, bf16
 
 struct PfTile {
-    int e, off, cnt, pad;          // expert, first entry position, entries (<= MT)
+    int e, off, cnt, pad;          // expert, first entry position, entries (at most the launch's tile size)
 };
 
 // Router GEMM logits = A . W^T over rows m0 .. m0+63 of A [a_rows x K] (bf16), bf16 weights.
@@ -74,6 +78,10 @@ struct PfExpArgs {
 
 WZY_DEV uint16_t f_to_bf16(float f) {                // hardware conversion, round to nearest even
     return __builtin_bit_cast(uint16_t, (__bf16) f);
+}
+// two of them in one conversion
+WZY_DEV uint32_t pack_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{a, b}, bf16x2_t));
 }
 WZY_DEV float bf16_bits_to_f(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 WZY_DEV uint32_t f_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
@@ -190,35 +198,35 @@ WZY_DEV float2_t e4m3x2(uint32_t s) {
     return float2_t{fminf(v.x, 480.0f), fminf(v.y, 480.0f)};
 }
 
-constexpr int EKB = 128;           // expert GEMM: weight chunk (k values) staged through LDS
+constexpr int ECB = 64;            // expert GEMM: code bytes of a weight row per chunk staged through LDS
 constexpr int EROWS = 256;         // weight rows per workgroup (8 waves x 32)
 constexpr int ETHR = 512;          // threads per expert workgroup
 enum { WF_FP4 = 0, WF_Q8 = 1 };    // weight formats of the expert GEMM
 
-// Bytes of one weight row per chunk (codes), and 16-byte pieces per thread to stage a chunk.
-template <int WF> constexpr int chunk_bytes() { return WF == WF_FP4 ? EKB / 2 : EKB; }
-template <int WF> constexpr int pieces_per_thread() { return chunk_bytes<WF>() * EROWS / 16 / ETHR; }
+// k values of a chunk; 16-byte pieces per thread to stage a chunk's codes, and pieces per row
+template <int WF> constexpr int chunk_k() { return WF == WF_FP4 ? 2 * ECB : ECB; }
+constexpr int ENP = ECB * EROWS / 16 / ETHR, EPPR = ECB / 16;
+static_assert(ENP == 2, "two staging pieces per thread");
 
 struct ExpLane {                   // per-thread view of one expert tile
     const uint8_t* crow0;          // staging: code bytes of the (row, 16-byte piece) slots, chunk 0
-    const uint8_t* crow1;
-    const uint8_t* crow2;          // (Q8 only)
-    const uint8_t* crow3;
-    const uint8_t* srow;           // staging (threads < 256): block scales of row `tid`, chunk 0
-    const uint16_t* ap;            // staging: activation row of entry sr (+ k offset sk)
+    uint32_t crow_d;               // from the first slot's row to the second's (128 local rows on)
+    const uint8_t* srow;           // staging: block scales of row tid / 2
     int lr;                        // the lane's weight row (local) = its B fragment column
-    int nk, cnt, row0, col, sr, sk;
-    bool a_ok;
+    int nk, cnt, row0, col, wr, wp;   // wr, wp: staging: LDS row and byte of the first code slot
     uint32_t sa;
     float ts;
 };
 
-template <int WF>
+// MTT: entries per tile; with 64 or 128 of them two workgroups share a CU's 160 KB.  144-byte activation rows
+// and code rows whose 16-byte pieces are permuted by the row (code_at) put the 16 rows that one LDS cycle
+// reads on different banks.
+template <int MTT>
 struct ExpLds {
-    uint16_t a[2][MT][EA_LD];                        // activation rows, one K step (64) per buffer
-    uint8_t b[2][EROWS][chunk_bytes<WF>() + 16];     // weight codes, one chunk (128 k) per buffer
-    uint2 s[2][EROWS];                               // the chunk's block scales per weight row (8 bytes)
-    int row[MT];                                     // A row of each tile entry
+    uint16_t a[2][MTT][EA_LD];                       // activation rows, one K step (64) per buffer
+    uint8_t b[2][EROWS][ECB];                        // weight codes, one chunk per buffer
+    uint2 s[2][EROWS][2];                            // block scales per weight row, two chunks per buffer
+    int row[MTT];                                    // A row of each tile entry
 };
 
 // MFMA B fragment from 8 Q8_0 codes (one k16 half) times their fp16 block scale, rounded to bf16
@@ -230,95 +238,120 @@ WZY_DEV bf16x8_t q8_frag(uint2 q, float sc) {
         const uint32_t w = i < 2 ? q.x : q.y;
         const float v0 = (float) (int8_t) (w >> (16 * (i & 1))) * sc;
         const float v1 = (float) (int8_t) (w >> (16 * (i & 1) + 8)) * sc;
-        b[i] = (uint32_t) f_to_bf16(v0) | ((uint32_t) f_to_bf16(v1) << 16);
+        b[i] = pack_bf16(v0, v1);
     }
     return __builtin_bit_cast(bf16x8_t, make_uint4(b[0], b[1], b[2], b[3]));
 }
 
-// K loop and epilogue of one tile with NMB active 32-entry row blocks.
-template <bool DOWN, int WF, int NMB>
-WZY_DEV void expert_tile(const PfExpArgs& a, const ExpLane c, ExpLds<WF>& L) {
-    constexpr int CB = chunk_bytes<WF>(), NP = pieces_per_thread<WF>(), PPR = CB / 16;
+// byte `at` of code row `row` in LDS (its 16-byte piece at / 16 lies at piece (at / 16) ^ (row / 4 % 4))
+WZY_DEV int code_at(int row, int at) { return at ^ ((row & 12) << 2); }
+
+// Block scales of two chunks (a pair) of a weight row: 16 e4m3 bytes or four fp16.  Threads 2 r and 2 r + 1
+// stage row r's halves: read two chunks at a time by two lanes a row, the scales cost an eighth of the cache
+// lines they do with one lane a row in every chunk (gate|up of 307 tokens 257 -> 212 us).
+template <int WF>
+WZY_DEV uint2 get_scales(const uint8_t* row, int pair, int K) {
+    const int hb = WF == WF_FP4 ? 8 : 4, half = threadIdx.x & 1;            // bytes per half = per chunk
+    const uint8_t* p = row + min((2 * pair + half) * hb, K / (chunk_k<WF>() / hb) - hb);   // an odd last chunk
+    if constexpr (WF == WF_FP4) return *(const uint2*) p;
+    else return make_uint2(*(const uint32_t*) p, 0u);
+}
+
+// staging registers: activation pieces of one K step, codes and scales of one weight chunk
+template <int NA>
+struct ExpA { u32x4_t v[NA]; };
+struct ExpW { u32x4_t q0, q1; };
+
+// K loop and epilogue of one tile with NMB active 32-entry row blocks.  Loads run DEPTH steps (activations)
+// and DEPTH chunks (weights) ahead, in register sets used in turn; the activations of a step are requested
+// before the weights of a chunk, so that waiting for them leaves the weights in flight.
+template <bool DOWN, int WF, int MTT, int NMB>
+WZY_DEV void expert_tile(const PfExpArgs& a, const ExpLane c, const uint16_t* const (&ap)[MTT / 64], ExpLds<MTT>& L) {
+    constexpr int SPC = chunk_k<WF>() / EK, NA = MTT / 64;          // steps per chunk, activation pieces per thread
+    constexpr int DEPTH = MTT == 64 ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
-    const int nkc = c.nk / (EKB / EK);                              // weight chunks
-    uint4 bq0 = make_uint4(0, 0, 0, 0), bq1 = bq0, bq2 = bq0, bq3 = bq0;
-    uint2 bs = make_uint2(0, 0);
+    const int nkc = c.nk / SPC;                                     // weight chunks
     f32x16_t acc[NMB];
 #pragma unroll
     for (int mb = 0; mb < NMB; ++mb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mb][i] = 0.f;
-
-    for (int kc = 0; kc < nkc; ++kc) {
-        const int bb = kc & 1;
-        const bool more_b = kc + 1 < nkc;
-        if (more_b) {                                               // next weight chunk, coalesced
-            const size_t o = (size_t) (kc + 1) * CB;
-            bq0 = *(const uint4*) (c.crow0 + o);
-            bq1 = *(const uint4*) (c.crow1 + o);
-            if constexpr (NP == 4) {
-                bq2 = *(const uint4*) (c.crow2 + o);
-                bq3 = *(const uint4*) (c.crow3 + o);
-            }
-            if (tid < EROWS) bs = *(const uint2*) (c.srow + (size_t) (kc + 1) * 8);
-        }
-        const uint2 sw = L.s[bb][c.lr];
+    ExpA<NA> xa[DEPTH];
+    ExpW xw[DEPTH];
+    // No load and no staging store of the loop is conditional: past the end the last step's and chunk's
+    // values are loaded and stored again, into buffers that nothing reads any more.  (A load under a
+    // condition makes the compiler wait for everything in flight wherever it waits at all.)
+    auto load_a = [&](ExpA<NA>& x, int ks) {
+        const size_t o = (size_t) min(ks, c.nk - 1) * EK;
 #pragma unroll
-        for (int st = 0; st < EKB / EK; ++st) {
-            const int ks = kc * (EKB / EK) + st;
-            const int ab = ks & 1;
-            uint4 xn[4];                                            // activations one step ahead
+        for (int i = 0; i < NA; ++i) x.v[i] = *(const u32x4_t*) (ap[i] + o);
+    };
+    auto load_w = [&](ExpW& x, int kc) {                            // coalesced
+        kc = min(kc, nkc - 1);
+        const size_t o = (size_t) kc * ECB;
+        x.q0 = *(const u32x4_t*) (c.crow0 + o);
+        x.q1 = *(const u32x4_t*) (c.crow0 + (o + c.crow_d));
+    };
+    uint2 xs;                                                       // the next pair's scales
+    // step 0 and chunk 0 are in LDS; the sets hold steps / chunks 1 .. DEPTH - 1
+    if constexpr (DEPTH == 2) {
+        load_a(xa[1], 1);
+        load_w(xw[1], 1);
+    }
+    // one chunk; PC = chunk parity, AP = parity of its first step
+    auto chunk = [&](auto pc, auto ap, int kc) {
+        constexpr int PC = decltype(pc)::value, AP = decltype(ap)::value;
+        const uint2 sw = L.s[(kc >> 1) & 1][c.lr][PC];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) xn[i] = make_uint4(0, 0, 0, 0);
-            if (ks + 1 < c.nk && c.a_ok) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) xn[i] = *(const uint4*) (c.ap + (size_t) (ks + 1) * EK + 8 * i);
-            }
-            bf16x8_t bfr[4];                                        // B fragments of k16 slices 4st .. 4st+3
+        for (int st = 0; st < SPC; ++st) {
+            const int ks = kc * SPC + st;
+            const int ab = (AP + st) & 1;
+            load_a(xa[DEPTH == 2 ? ab : 0], ks + DEPTH);            // set ab held step ks, stored one step ago
+            if (st == 0) load_w(xw[DEPTH == 2 ? PC : 0], kc + DEPTH);
+            if (st == 0 && PC == 0) xs = get_scales<WF>(c.srow, (kc >> 1) + 1, a.K);
+            const uint32_t sv = st ? sw.y : sw.x;
+            float sc[4];                                            // per k16 slice: its block scale
             if constexpr (WF == WF_FP4) {
-                // 8 code bytes and one e4m3 scale per slice
-                const uint32_t sv = st ? sw.y : sw.x;
                 const float2_t sc01 = e4m3x2(sv), sc23 = e4m3x2(sv >> 16);
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const uint2 qq = *(const uint2*) &L.b[bb][c.lr][st * 32 + 8 * kk];
-                    const float scv = kk == 0 ? sc01.x : kk == 1 ? sc01.y : kk == 2 ? sc23.x : sc23.y;
-                    bfr[kk] = fp4_frag(qq.x, qq.y, c.sa, scv);
-                }
+                sc[0] = sc01.x; sc[1] = sc01.y; sc[2] = sc23.x; sc[3] = sc23.y;
             } else {
-                // 16 code bytes per slice (this lane's 8 at byte 8h); one fp16 scale per two slices
-                const uint32_t sv = st ? sw.y : sw.x;
-                const float s0 = h16_to_f((uint16_t) sv), s1 = h16_to_f((uint16_t) (sv >> 16));
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    const uint2 qq = *(const uint2*) &L.b[bb][c.lr][st * 64 + 16 * kk + 8 * h];
-                    bfr[kk] = q8_frag(qq, kk < 2 ? s0 : s1);
-                }
+                sc[0] = sc[1] = h16_to_f((uint16_t) sv);
+                sc[2] = sc[3] = h16_to_f((uint16_t) (sv >> 16));
             }
 #pragma unroll
             for (int kk = 0; kk < 4; ++kk) {
+                // B fragment of the slice: 8 bytes of the row, or this lane's 8 of 16 (Q8_0)
+                const uint2 qq = *(const uint2*) &L.b[PC][c.lr][code_at(c.lr, WF == WF_FP4 ? st * 32 + 8 * kk : 16 * kk + 8 * h)];
+                const bf16x8_t bv = WF == WF_FP4 ? fp4_frag(qq.x, qq.y, c.sa, sc[kk]) : q8_frag(qq, sc[kk]);
 #pragma unroll
                 for (int mb = 0; mb < NMB; ++mb) {
                     const bf16x8_t av = *(const bf16x8_t*) &L.a[ab][mb * 32 + (lane & 31)][kk * 16 + h * 8];
-                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bfr[kk], acc[mb], 0, 0, 0);
+                    acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[mb], 0, 0, 0);
                 }
             }
-            if (ks + 1 < c.nk) {
+            {
+                const ExpA<NA>& x = xa[DEPTH == 2 ? ab ^ 1 : 0];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) *(uint4*) &L.a[ab ^ 1][c.sr][c.sk + 8 * i] = xn[i];
+                for (int i = 0; i < NA; ++i) *(u32x4_t*) &L.a[ab ^ 1][(tid >> 3) + 64 * i][(tid & 7) * 8] = x.v[i];
             }
-            if (st == EKB / EK - 1 && more_b) {                     // the next chunk into the other buffer
-                *(uint4*) &L.b[bb ^ 1][tid / PPR][(tid % PPR) * 16] = bq0;
-                *(uint4*) &L.b[bb ^ 1][(ETHR + tid) / PPR][(tid % PPR) * 16] = bq1;
-                if constexpr (NP == 4) {
-                    *(uint4*) &L.b[bb ^ 1][(2 * ETHR + tid) / PPR][(tid % PPR) * 16] = bq2;
-                    *(uint4*) &L.b[bb ^ 1][(3 * ETHR + tid) / PPR][(tid % PPR) * 16] = bq3;
-                }
-                if (tid < EROWS) L.s[bb ^ 1][tid] = bs;
+            if (st == SPC - 1) {                                    // the next chunk into the other buffer
+                const ExpW& x = xw[DEPTH == 2 ? PC ^ 1 : 0];
+                *(u32x4_t*) &L.b[PC ^ 1][c.wr][c.wp] = x.q0;
+                *(u32x4_t*) &L.b[PC ^ 1][c.wr + 128][c.wp] = x.q1;
+                if (PC == 1) L.s[((kc >> 1) + 1) & 1][tid >> 1][tid & 1] = xs;
             }
             __syncthreads();
         }
+    };
+    using P0 = std::integral_constant<int, 0>;
+    using P1 = std::integral_constant<int, 1>;
+    using PS = std::integral_constant<int, SPC & 1>;                // parity of an odd chunk's first step
+    int kc = 0;
+    for (; kc + 1 < nkc; kc += 2) {
+        chunk(P0{}, P0{}, kc);
+        chunk(P1{}, PS{}, kc + 1);
     }
+    if (kc < nkc) chunk(P0{}, P0{}, kc);
 
     // acc[mb][i] = C[entry mb*32 + 8*(i/4) + 4*h + i%4][column lane%32 of the wave's weight block]
     const bool gate_lane = (lane & 16) == 0;
@@ -344,27 +377,25 @@ WZY_DEV void expert_tile(const PfExpArgs& a, const ExpLane c, ExpLds<WF>& L) {
     }
 }
 
-// Routed-expert GEMM.  Workgroup = one expert tile (<= 256 entries) x 256 weight rows, 8 waves; wave
+// Routed-expert GEMM.  Workgroup = one expert tile (up to MTT entries) x 256 weight rows, 8 waves; wave
 // w owns one 32-row weight block (gate|up: 16 gate rows j0+16w.. in columns 0..15 and the matching
 // 16 up rows in columns 16..31, paired for SwiGLU across lanes l, l^16; down: rows n0+32w .. +31)
 // for all active 32-entry row blocks of the tile (the count selects a specialised loop), so each
-// dequantised B fragment feeds up to 8 MFMAs.  Weight codes move in 128-k chunks: each row's code
-// bytes are read as 16-byte pieces by adjacent threads (whole 64-byte segments), one chunk ahead,
-// into LDS; each lane then takes its row's bytes per k16 slice from LDS and dequantises them into
-// its MFMA B fragment.  The activation rows of the tile are staged in LDS one 64-k step ahead and
-// shared by the eight waves.  Workgroups are numbered so that consecutive workgroups of one XCD take
-// the column blocks of one tile (its activation rows stay in that XCD's L2).  The tensor scale is
+// dequantised B fragment feeds up to MTT / 32 MFMAs.  Weight codes move in chunks of 64 bytes a row (128 k
+// values of NVFP4, 64 of Q8_0): read as 16-byte pieces by adjacent threads (whole 64-byte segments), one
+// chunk ahead, into LDS; each lane then takes its row's bytes per k16 slice from LDS and dequantises them
+// into its MFMA B fragment.  The activation rows of the tile are staged in LDS one 64-k step ahead and
+// shared by the eight waves.  Workgroups are numbered so that one XCD takes the column blocks of a tile
+// back to back, and pairs of consecutive tiles (an expert's tiles share its weights).  The tensor scale is
 // applied to the fp32 accumulators.  WF_Q8 with a null tile list runs the dense shared-expert
-// GEMMs over consecutive blocks of token rows.
-template <bool DOWN, int WF>
-__global__ void __launch_bounds__(ETHR, 1) pf_expert_kernel(PfExpArgs a) {
-    constexpr int CB = chunk_bytes<WF>(), NP = pieces_per_thread<WF>(), PPR = CB / 16;
-    __shared__ __align__(16) ExpLds<WF> L;
+// GEMMs over consecutive blocks of token rows.  An entry's sums do not depend on its tile or on MTT.
+template <bool DOWN, int WF, int MTT>
+WZY_DEV void expert_block(const PfExpArgs& a, int bx, ExpLds<MTT>& L) {
     const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int bx = blockIdx.x, jx = bx >> 3;
-    const int ti = (jx / a.gx) * 8 + (bx & 7), nb = jx % a.gx;
-    const bool dense = a.tiles == nullptr;
+    const int jx = bx >> 3, u = jx / a.gx, nb = jx % a.gx;
+    const int ti = (u >> 1) * 16 + (bx & 7) * 2 + (u & 1);
+    const bool dense = WF == WF_Q8;
     if (ti >= (dense ? (a.a_rows + a.dense_mt - 1) / a.dense_mt : *a.n_tiles)) return;   // workgroup-uniform
     ExpLane c;
     int e = 0;
@@ -377,7 +408,7 @@ __global__ void __launch_bounds__(ETHR, 1) pf_expert_kernel(PfExpArgs a) {
         c.row0 = t.off;
         e = t.e;
     }
-    if (tid < MT)
+    if (tid < MTT)
         L.row[tid] = tid < c.cnt ? ((DOWN || dense) ? c.row0 + tid : a.tok[c.row0 + tid] / a.topk) : 0;
     const uint8_t* rec = a.experts + (size_t) e * a.rec;
     // local weight row lr = 32w + column -> weight row: gate|up: columns 0..15 gate rows
@@ -407,41 +438,52 @@ __global__ void __launch_bounds__(ETHR, 1) pf_expert_kernel(PfExpArgs a) {
     } else {
         c.ts = 1.0f;
     }
-    const int pp = (tid % PPR) * 16;
-    c.crow0 = code_row(tid / PPR) + pp;
-    c.crow1 = code_row((ETHR + tid) / PPR) + pp;
-    c.crow2 = NP == 4 ? code_row((2 * ETHR + tid) / PPR) + pp : c.crow0;
-    c.crow3 = NP == 4 ? code_row((3 * ETHR + tid) / PPR) + pp : c.crow0;
-    c.srow = scale_row(tid & (EROWS - 1));
+    const int pp = (tid % EPPR) * 16;
+    c.crow0 = code_row(tid / EPPR) + pp;
+    // 128 local rows are four wave blocks: 128 down rows, or 64 rows of the same matrix of gate|up
+    c.crow_d = (DOWN ? 128u : 64u) * (uint32_t) (WF == WF_FP4 ? a.K / 2 : a.K);
+    c.srow = scale_row(tid >> 1);
     c.nk = a.K / EK;
     c.sa = 4u * h;
     // weight chunk 0
-    *(uint4*) &L.b[0][tid / PPR][pp] = *(const uint4*) c.crow0;
-    *(uint4*) &L.b[0][(ETHR + tid) / PPR][pp] = *(const uint4*) c.crow1;
-    if constexpr (NP == 4) {
-        *(uint4*) &L.b[0][(2 * ETHR + tid) / PPR][pp] = *(const uint4*) c.crow2;
-        *(uint4*) &L.b[0][(3 * ETHR + tid) / PPR][pp] = *(const uint4*) c.crow3;
-    }
-    if (tid < EROWS) L.s[0][tid] = *(const uint2*) c.srow;
+    c.wr = tid / EPPR;
+    c.wp = code_at(c.wr, pp);                                       // row wr + 128 has the same permutation
+    *(u32x4_t*) &L.b[0][c.wr][c.wp] = *(const u32x4_t*) c.crow0;
+    *(u32x4_t*) &L.b[0][c.wr + 128][c.wp] = *(const u32x4_t*) (c.crow0 + c.crow_d);
+    L.s[0][tid >> 1][tid & 1] = get_scales<WF>(c.srow, 0, a.K);
     __syncthreads();
-    c.sr = tid >> 1;                                                // staging: entry sr, k sk .. sk+31
-    c.sk = (tid & 1) * 32;
-    c.a_ok = c.sr < c.cnt;
-    c.ap = a.a + (size_t) L.row[c.sr] * a.K + c.sk;
+    // activation staging: eight lanes read a row's 128 bytes of a step; thread -> rows tid / 8 + 64 i.  Slots
+    // past the tile's entries stage row 0 of the operand: their products are never stored.
+    constexpr int NA = MTT / 64;
+    const uint16_t* ap[NA];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        *(uint4*) &L.a[0][c.sr][c.sk + 8 * i] = c.a_ok ? *(const uint4*) (c.ap + 8 * i) : make_uint4(0, 0, 0, 0);
-    __syncthreads();
-    switch ((c.cnt + 31) >> 5) {                                    // workgroup-uniform
-        case 1: expert_tile<DOWN, WF, 1>(a, c, L); break;
-        case 2: expert_tile<DOWN, WF, 2>(a, c, L); break;
-        case 3: expert_tile<DOWN, WF, 3>(a, c, L); break;
-        case 4: expert_tile<DOWN, WF, 4>(a, c, L); break;
-        case 5: expert_tile<DOWN, WF, 5>(a, c, L); break;
-        case 6: expert_tile<DOWN, WF, 6>(a, c, L); break;
-        case 7: expert_tile<DOWN, WF, 7>(a, c, L); break;
-        default: expert_tile<DOWN, WF, 8>(a, c, L); break;
+    for (int i = 0; i < NA; ++i) {
+        const int sr = (tid >> 3) + 64 * i;
+        ap[i] = a.a + (size_t) L.row[sr] * a.K + (tid & 7) * 8;
+        *(u32x4_t*) &L.a[0][sr][(tid & 7) * 8] = *(const u32x4_t*) ap[i];
     }
+    __syncthreads();
+    const int nmb = (c.cnt + 31) >> 5;                              // workgroup-uniform
+    if constexpr (MTT == 64) {
+        if (nmb == 1) expert_tile<DOWN, WF, MTT, 1>(a, c, ap, L);
+        else expert_tile<DOWN, WF, MTT, 2>(a, c, ap, L);
+    } else {
+        switch (nmb) {
+            case 1: expert_tile<DOWN, WF, MTT, 1>(a, c, ap, L); break;
+            case 2: expert_tile<DOWN, WF, MTT, 2>(a, c, ap, L); break;
+            case 3: expert_tile<DOWN, WF, MTT, 3>(a, c, ap, L); break;
+            default: expert_tile<DOWN, WF, MTT, 4>(a, c, ap, L); break;
+        }
+    }
+}
+
+// Routed tiles `r`, or dense blocks `d` of the shared expert, or both in one launch (the first nd
+// workgroups take the dense blocks): a short chunk's few dense blocks then run beside the routed ones.
+template <bool DOWN, int MTT>
+__global__ void __launch_bounds__(ETHR, 4) pf_expert_kernel(PfExpArgs r, PfExpArgs d, int nd) {
+    __shared__ __align__(16) ExpLds<MTT> L;
+    if ((int) blockIdx.x < nd) expert_block<DOWN, WF_Q8, MTT>(d, blockIdx.x, L);
+    else expert_block<DOWN, WF_FP4, MTT>(r, blockIdx.x - nd, L);
 }
 
 // x fp32 -> bf16; workgroup 0 also clears the per-expert entry cursors
@@ -452,8 +494,7 @@ __global__ void __launch_bounds__(256) pf_cvt_kernel(const float* __restrict__ x
     const size_t i = ((size_t) blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= n) return;
     const float4 v = *(const float4*) (x + i);
-    *(uint2*) (xb + i) = make_uint2(f_to_bf16(v.x) | ((uint32_t) f_to_bf16(v.y) << 16),
-                                    f_to_bf16(v.z) | ((uint32_t) f_to_bf16(v.w) << 16));
+    *(uint2*) (xb + i) = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w));
 }
 
 // one wave per token: routing of its logits row and the shared-expert gate
@@ -509,13 +550,15 @@ __global__ void __launch_bounds__(256) pf_hist_kernel(const int* __restrict__ id
 }
 
 // one workgroup: exclusive scans of the entry counts and of the tiles per expert -> each expert's
-// first entry position and its MT-entry tiles
-__global__ void __launch_bounds__(1024) pf_tiles_kernel(const int* __restrict__ cnt, int E, int* __restrict__ exp_off,
-                                                        PfTile* __restrict__ tiles, int* __restrict__ n_tiles) {
+// first entry position and its tiles of at most mt entries (as many as needed, of equal size rounded up to
+// whole 32-entry row blocks)
+__global__ void __launch_bounds__(1024) pf_tiles_kernel(const int* __restrict__ cnt, int E, int mt,
+                                                        int* __restrict__ exp_off, PfTile* __restrict__ tiles,
+                                                        int* __restrict__ n_tiles) {
     __shared__ uint64_t s_w[16];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int c = tid < E ? cnt[tid] : 0;
-    const int nt = (c + MT - 1) / MT;
+    const int nt = (c + mt - 1) / mt;
     const uint64_t v = ((uint64_t) c << 24) | (uint64_t) nt;       // both sums in one scan
     uint64_t s = v;
 #pragma unroll
@@ -531,7 +574,8 @@ __global__ void __launch_bounds__(1024) pf_tiles_kernel(const int* __restrict__ 
     const int off = (int) (ex >> 24), toff = (int) (ex & 0xFFFFFFu);
     if (tid < E) {
         exp_off[tid] = off;
-        for (int q = 0; q < nt; ++q) tiles[toff + q] = PfTile{tid, off + q * MT, min(MT, c - q * MT), 0};
+        const int per = nt > 0 ? ((c + nt - 1) / nt + 31) & ~31 : 0;     // <= mt, (nt - 1) * per < c
+        for (int q = 0; q < nt; ++q) tiles[toff + q] = PfTile{tid, off + q * per, min(per, c - q * per), 0};
     }
     if (tid == 1023) *n_tiles = (int) ((base + s) & 0xFFFFFFu);
 }
@@ -592,14 +636,22 @@ struct PfWs {
     uint16_t* xb; float* logits; float* sg; int* ids; float* wts;
     int* cursor; int* exp_off; int* wg_base; int* rank; int* ent_idx; int* ent_pos; PfTile* tiles; int* n_tiles;
     uint16_t* act; uint16_t* sh_act; float* y;
-    int max_tiles, n_wg;
+    int mt, max_tiles, n_wg;
 };
+
+// Entries per expert tile.  Both sizes put two workgroups on a CU, so that one computes while the other waits
+// for a K step (one workgroup a CU with 256-entry tiles: 307 tokens 324 + 179 us gate|up + down, now 212 +
+// 116; 8,192 tokens 490 + 533, now 483 + 512).  64-entry tiles stage half the rows and load two steps ahead;
+// beyond 60 entries an expert too many experts need two of them (512 experts top-10, whole block: 59 entries
+// 565 us with 64 against 592 with 128, 68 entries 650 against 632).
+int pf_tile_entries(size_t n_ent, int E) { return n_ent <= (size_t) 60 * E ? 64 : 128; }
 
 PfWs pf_ws_carve(void* base, size_t cap, int D, int F, int E, int K, int N, size_t* need) {
     Arena a(base, cap);
     PfWs w;
     const size_t n_ent = (size_t) N * K;
-    w.max_tiles = (int) (n_ent / MT + E);
+    w.mt = pf_tile_entries(n_ent, E);
+    w.max_tiles = (int) (n_ent / w.mt + E);
     w.xb = a.take<uint16_t>((size_t) N * D);
     w.logits = a.take<float>((size_t) N * E);
     w.sg = a.take<float>(N);
@@ -621,16 +673,16 @@ PfWs pf_ws_carve(void* base, size_t cap, int D, int F, int E, int K, int N, size
     return w;
 }
 
+// workgroups of `tiles` tiles x gx column blocks (whole rounds of 8 XCDs x 2 tiles)
+unsigned expert_grid(int tiles, int gx) { return (unsigned) (gx * ((tiles + 15) / 16) * 16); }
+
+// the routed tiles (max_tiles > 0), the dense blocks (d.a_rows > 0), or both in one launch
 template <bool DOWN>
-void launch_expert(const PfExpArgs& a, int max_tiles, hipStream_t st) {
-    const unsigned n = (unsigned) (a.gx * ((max_tiles + 7) / 8) * 8);
-    hipLaunchKernelGGL((pf_expert_kernel<DOWN, WF_FP4>), dim3(n), dim3(ETHR), 0, st, a);
-}
-template <bool DOWN>
-void launch_dense_q8(const PfExpArgs& a, hipStream_t st) {
-    const int nt = (a.a_rows + a.dense_mt - 1) / a.dense_mt;
-    const unsigned n = (unsigned) (a.gx * ((nt + 7) / 8) * 8);
-    hipLaunchKernelGGL((pf_expert_kernel<DOWN, WF_Q8>), dim3(n), dim3(ETHR), 0, st, a);
+void launch_expert(int mt, const PfExpArgs& r, int max_tiles, const PfExpArgs& d, hipStream_t st) {
+    const unsigned nd = d.a_rows > 0 ? expert_grid((d.a_rows + d.dense_mt - 1) / d.dense_mt, d.gx) : 0;
+    const unsigned n = nd + (max_tiles > 0 ? expert_grid(max_tiles, r.gx) : 0);
+    if (mt == 64) hipLaunchKernelGGL((pf_expert_kernel<DOWN, 64>), dim3(n), dim3(ETHR), 0, st, r, d, (int) nd);
+    else hipLaunchKernelGGL((pf_expert_kernel<DOWN, 128>), dim3(n), dim3(ETHR), 0, st, r, d, (int) nd);
 }
 
 }  // namespace
@@ -647,6 +699,10 @@ extern "C" size_t wzy_moe_prefill_workspace_bytes(int n_embd, int n_ff, int n_ex
 namespace {
 
 constexpr int PF_N_STAGES = 8;     // timing groups of pf_enqueue
+// Rows from which the shared expert has launches of its own.  Below, its few dense blocks run beside the
+// routed tiles (307 tokens: 58 + 50 us as launches of 12 and 16 workgroups, under 10 beside them; 6,000 tokens
+// 933 us apart, 907 together); from here on both take the same time.
+constexpr int PF_APART_ROWS = 8192;
 
 int pf_check(const wzy_moe_weights* w, int N) {
     WZY_REQUIRE(w, "wzy_moe_prefill: null weights");
@@ -699,49 +755,42 @@ void pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, co
     mark(3);
     hipLaunchKernelGGL(pf_hist_kernel, dim3((unsigned) ws.n_wg), dim3(256), 0, st, ws.ids, n_ent, E, ws.cursor,
                        ws.wg_base, ws.rank);
-    hipLaunchKernelGGL(pf_tiles_kernel, dim3(1), dim3(1024), 0, st, ws.cursor, E, ws.exp_off, ws.tiles, ws.n_tiles);
+    hipLaunchKernelGGL(pf_tiles_kernel, dim3(1), dim3(1024), 0, st, ws.cursor, E, ws.mt, ws.exp_off, ws.tiles, ws.n_tiles);
     hipLaunchKernelGGL(pf_scatter_kernel, dim3((unsigned) ((n_ent + 255) / 256)), dim3(256), 0, st, ws.ids, ws.rank,
                        ws.wg_base, ws.exp_off, n_ent, K, E, ws.ent_idx, ws.ent_pos);
-    // shared expert gate|up + SwiGLU, then down -> comb = sigmoid(sg) * shared (dense Q8_0 tiles)
+    // shared expert (dense Q8_0 blocks): gate|up + SwiGLU, then down -> comb = sigmoid(sg) * shared; routed
+    // experts: gate|up + SwiGLU per tile, down per tile, then the per-token weighted sum
+    PfExpArgs sgu{}, sdn{}, rgu{}, rdn{};
+    sgu.experts = w->experts; sgu.K = D; sgu.F = F; sgu.gx = F / 128;
+    sgu.a_rows = N; sgu.dense_mt = ws.mt; sgu.a = ws.xb;
+    sgu.w = (const int8_t*) w->sh_gate_q; sgu.ws = (const uint16_t*) w->sh_gate_s;
+    sgu.w2 = (const int8_t*) w->sh_up_q; sgu.ws2 = (const uint16_t*) w->sh_up_s;
+    sgu.act = ws.sh_act; sgu.ld_out = F;
+    sdn.experts = w->experts; sdn.K = F; sdn.gx = D / EROWS;
+    sdn.a_rows = N; sdn.dense_mt = ws.mt; sdn.a = ws.sh_act;
+    sdn.w = (const int8_t*) w->sh_down_q; sdn.ws = (const uint16_t*) w->sh_down_s;
+    sdn.y = comb; sdn.ld_out = D; sdn.sg = ws.sg;
+    rgu.experts = w->experts; rgu.rec = o.rec; rgu.codes_off = o.gu_codes; rgu.scales_off = o.gu_scales;
+    rgu.tail_off = o.tail; rgu.K = D; rgu.F = F; rgu.gx = F / 128;
+    rgu.tiles = ws.tiles; rgu.n_tiles = ws.n_tiles;
+    rgu.a = ws.xb; rgu.tok = ws.ent_idx; rgu.topk = K;
+    rgu.act = ws.act; rgu.ld_out = F;
+    rdn.experts = w->experts; rdn.rec = o.rec; rdn.codes_off = o.dn_codes; rdn.scales_off = o.dn_scales;
+    rdn.tail_off = o.tail; rdn.K = F; rdn.F = 0; rdn.gx = D / EROWS;
+    rdn.tiles = ws.tiles; rdn.n_tiles = ws.n_tiles;
+    rdn.a = ws.act; rdn.tok = nullptr; rdn.topk = K;
+    rdn.y = ws.y; rdn.ld_out = D;
+    const bool apart = N >= PF_APART_ROWS;
+    const PfExpArgs none{};
     mark(4);
-    {
-        PfExpArgs a{};
-        a.experts = w->experts; a.K = D; a.F = F; a.gx = F / 128;
-        a.a_rows = N; a.dense_mt = MT / 2; a.a = ws.xb;     // 128-row blocks: F/128 x N/128 workgroups
-        a.w = (const int8_t*) w->sh_gate_q; a.ws = (const uint16_t*) w->sh_gate_s;
-        a.w2 = (const int8_t*) w->sh_up_q; a.ws2 = (const uint16_t*) w->sh_up_s;
-        a.act = ws.sh_act; a.ld_out = F;
-        launch_dense_q8<false>(a, st);
-    }
+    if (apart) launch_expert<false>(ws.mt, none, 0, sgu, st);
     mark(5);
-    {
-        PfExpArgs b{};
-        b.experts = w->experts; b.K = F; b.gx = D / EROWS;
-        b.a_rows = N; b.dense_mt = MT; b.a = ws.sh_act;
-        b.w = (const int8_t*) w->sh_down_q; b.ws = (const uint16_t*) w->sh_down_s;
-        b.y = comb; b.ld_out = D; b.sg = ws.sg;
-        launch_dense_q8<true>(b, st);
-    }
-    // routed experts: gate|up + SwiGLU per tile, down per tile, then the per-token weighted sum
+    if (apart) launch_expert<true>(ws.mt, none, 0, sdn, st);
     mark(6);
-    {
-        PfExpArgs a{};
-        a.experts = w->experts; a.rec = o.rec; a.codes_off = o.gu_codes; a.scales_off = o.gu_scales;
-        a.tail_off = o.tail; a.K = D; a.F = F; a.gx = F / 128;
-        a.tiles = ws.tiles; a.n_tiles = ws.n_tiles;
-        a.a = ws.xb; a.tok = ws.ent_idx; a.topk = K;
-        a.act = ws.act; a.ld_out = F;
-        launch_expert<false>(a, ws.max_tiles, st);
-    }
+    launch_expert<false>(ws.mt, rgu, ws.max_tiles, apart ? none : sgu, st);
     mark(7);
     {
-        PfExpArgs b{};
-        b.experts = w->experts; b.rec = o.rec; b.codes_off = o.dn_codes; b.scales_off = o.dn_scales;
-        b.tail_off = o.tail; b.K = F; b.F = 0; b.gx = D / 256;
-        b.tiles = ws.tiles; b.n_tiles = ws.n_tiles;
-        b.a = ws.act; b.tok = nullptr; b.topk = K;
-        b.y = ws.y; b.ld_out = D;
-        launch_expert<true>(b, ws.max_tiles, st);
+        launch_expert<true>(ws.mt, rdn, ws.max_tiles, apart ? none : sdn, st);
         const dim3 cg((unsigned) ((D / 4 + 255) / 256), (unsigned) N);
         if (K == 10)
             hipLaunchKernelGGL((pf_combine_kernel<10, true>), cg, dim3(256), 0, st, ws.y, ws.ent_pos, ws.wts, K, D, comb);
