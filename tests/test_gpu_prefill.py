@@ -129,6 +129,30 @@ def test_gemm_bf16_parity(wz, orc, gpu, M, N, K, kind, out):
         assert (got[:, N:] == 0xABCD).all(), "wrote past N"
 
 
+def test_gemm_tile_sizes_agree(wz, gpu):
+    """The GEMM takes 64- or 128-wide tiles and one or several k steps in flight by the launch's tile count;
+    an output element's bits depend on none of it: rows of a longer product equal the same rows of
+    shorter ones (1 to 1,500 rows x 1,100 columns: 9 to 108 tiles of 128; x 6,100: 48 to 576)."""
+    print("case gemm_tile_sizes", flush=True)
+    rng = np.random.default_rng(12)
+    M, K = 1500, 320
+    a = DA.from_numpy(bf16_bits(rng.normal(0, 1, (M, K))))
+    for N in (1100, 6100):
+        wq = DA.from_numpy(rng.integers(-127, 128, N * K).astype(np.int8))
+        ws = DA.from_numpy(rng.uniform(0.0005, 0.002, N * K // 32).astype(np.float16).view(np.uint16))
+        wb = DA.from_numpy(bf16_bits(rng.normal(0, 0.05, N * K)))
+        for q8 in (True, False):
+            ref = None
+            for m in (M, 1, 63, 65, 700, 1281):
+                y = DA((m, N), np.float32)
+                wz.wzy_gemm_bf16(a.ptr, K, m, K, wq.ptr if q8 else None, ws.ptr if q8 else None,
+                                 None if q8 else wb.ptr, N, y.ptr, None, N, None)
+                wz.wzy_device_sync()
+                got = y.numpy()
+                ref = got if ref is None else ref
+                np.testing.assert_array_equal(got, ref[:m])
+
+
 # ---- whole chunks against the oracle, teacher-forced on the discrete decisions ---------------------
 def router_gaps(dm, w, x):
     """top_k-th minus (top_k+1)-th router logit of bf16(x) rows (fp64 sums)"""

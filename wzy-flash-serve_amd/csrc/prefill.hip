@@ -1,7 +1,7 @@
 // prefill.hip -- kernels of the chunked prefill (B prompt cells per launch sequence) on gfx950.
 //
 //  pf_gemm       every dense projection of the chunk on bf16 MFMA (v_mfma_f32_32x32x16_bf16):
-//                128 x 128 output tiles, K in steps of 64 through two LDS buffers; Q8_0 weights are
+//                128 x 128 or 64 x 64 output tiles, K in steps of 64 through LDS; Q8_0 weights are
 //                dequantised (code * fp16 scale, rounded to bf16) on their way into LDS, bf16
 //                weights copied.  Workgroups are numbered so that the eight XCDs take interleaved row
 //                tiles and each runs all weight tiles of its row tile back to back.  A few bf16
@@ -31,7 +31,10 @@
 using namespace wzy;
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x3_t __attribute__((ext_vector_type(3)));
 typedef int i32x2_t __attribute__((ext_vector_type(2)));
@@ -40,42 +43,42 @@ typedef int i32x4_t __attribute__((ext_vector_type(4)));
 namespace {
 
 WZY_DEV uint16_t f_to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16) f); }   // nearest even
-WZY_DEV uint32_t pack_bf16(float a, float b) { return (uint32_t) f_to_bf16(a) | ((uint32_t) f_to_bf16(b) << 16); }
+WZY_DEV uint32_t pack_bf16(float a, float b) {                                              // both in one conversion
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2_t{a, b}, bf16x2_t));
+}
 
 // ---------------------------------------------------------------------------------------------
 // dense GEMM
 // ---------------------------------------------------------------------------------------------
-constexpr int GM = 128, GN = 128, GK = 64, GLD = GK + 8;   // tile rows, weight rows, k step, LDS row (bf16)
+constexpr int GK = 64, GLD = GK + 8;                         // k step, LDS row (bf16)
 
 struct GemmArgs {
     PfGemm g;
     int mt, nt;
 };
 
-// 32 Q8_0 codes (one block, c0 | c1) times their fp16 scale, rounded to bf16, as four 16-byte pieces
+// eight Q8_0 codes times their fp16 scale, rounded to bf16
 WZY_DEV uint4 q8_quarter_bf16(uint32_t a, uint32_t b, float sc) {
     return make_uint4(pack_bf16((float) (int8_t) a * sc, (float) (int8_t) (a >> 8) * sc),
                       pack_bf16((float) (int8_t) (a >> 16) * sc, (float) (int8_t) (a >> 24) * sc),
                       pack_bf16((float) (int8_t) b * sc, (float) (int8_t) (b >> 8) * sc),
                       pack_bf16((float) (int8_t) (b >> 16) * sc, (float) (int8_t) (b >> 24) * sc));
 }
-WZY_DEV void q8_block_bf16(uint4 c0, uint4 c1, float sc, uint4& o0, uint4& o1, uint4& o2, uint4& o3) {
-    o0 = q8_quarter_bf16(c0.x, c0.y, sc);
-    o1 = q8_quarter_bf16(c0.z, c0.w, sc);
-    o2 = q8_quarter_bf16(c1.x, c1.y, sc);
-    o3 = q8_quarter_bf16(c1.z, c1.w, sc);
-}
 
 // UM: the HC up projection with the stream mean as its epilogue.  Tile column n holds stream
 // c = n % 4 of position d = n / 4 (weight row c * um_d + d), so a row's four stream gates sit in
 // one lane quad and are combined there in stream order.
+// T: tile side; a wave holds a quarter of the tile.  An element's sum runs over k in the same order and
+// instructions whatever T.
 // SB: one LDS buffer (37 KB), so four workgroups share a CU (three with the UM epilogue, whose
-// registers allow no more); the next k step still loads into
-// registers during the MFMAs, and a second barrier per step guards the buffer.  Launches with at
-// least 512 tiles use it; smaller ones keep two buffers (74 KB, two workgroups per CU).
-template <bool UM, bool SB>
-__global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : 2) pf_gemm_kernel(GemmArgs ga) {
-    constexpr int NBUF = SB ? 1 : 2;
+// registers allow no more); the next k step still loads into registers during the MFMAs, and a second
+// barrier per step guards the buffer.  Launches with at least 512 tiles use it; smaller ones keep two.
+// With a thread's 64 bytes of one row per step replaced by whole rows per eight lanes (below), 8,192 x 6,144 x
+// 2,048 took 338 -> 275 us from Q8_0 and 295 -> 260 us from bf16 (791 TFLOP/s), 250 x 12,288 x 2,048 53 -> 31.
+template <int T, bool UM, bool SB, bool Q8>
+__global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : T == 64 ? (Q8 ? 4 : 3) : 2) pf_gemm_kernel(GemmArgs ga) {
+    constexpr int GM = T, GN = T, NB = T / 64;                     // tile; 32 x 32 blocks per wave and side
+    constexpr int NBUF = SB ? 1 : 2, NA = GM / 32, NW = Q8 ? GN / 64 : GN / 32;
     __shared__ __align__(16) uint16_t sAW[NBUF * (GM + GN) * GLD];
     uint16_t (*const sA)[GM][GLD] = (uint16_t (*)[GM][GLD]) sAW;
     uint16_t (*const sW)[GN][GLD] = (uint16_t (*)[GN][GLD]) (sAW + NBUF * GM * GLD);
@@ -96,90 +99,110 @@ __global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : 2) pf_gemm_kernel(Gem
         ni = b % ga.nt;
     }
     const int m0 = mi * GM, n0 = ni * GN;
-    const int sr = tid >> 1, kh = (tid & 1) * 32;                  // staging: row sr, k kh .. kh+31
     const int nk = g.K / GK / max(g.ksplit, 1);                    // k steps of this launch's range
     const size_t k0 = (size_t) ksp * nk * GK;
-    const uint16_t* ap = g.a + (size_t) min(m0 + sr, g.M - 1) * g.lda + k0 + kh;
-    size_t wr = (size_t) min(n0 + sr, g.N - 1);
-    if (UM) wr = (wr & 3) * (size_t) g.um_d + (wr >> 2);
-    const bool q8 = g.wq != nullptr;
-    const int8_t* wqp = q8 ? g.wq + wr * g.K + k0 + kh : nullptr;
-    const uint16_t* wsp = q8 ? g.ws + wr * (g.K / 32) + (k0 + kh) / 32 : nullptr;
-    const uint16_t* wbp = q8 ? nullptr : g.wb + wr * g.K + k0 + kh;
-
-    // staging registers are scalars: arrays captured by a lambda would live in scratch memory
-    uint4 ra0, ra1, ra2, ra3, rw0, rw1, rw2 = make_uint4(0, 0, 0, 0), rw3 = rw2;
-    float rs = 0.f;
-#define PF_GEMM_LOAD(ks)                                                         \
-    {                                                                            \
-        const size_t o_ = (size_t) (ks) * GK;                                    \
-        ra0 = *(const uint4*) (ap + o_);                                         \
-        ra1 = *(const uint4*) (ap + o_ + 8);                                     \
-        ra2 = *(const uint4*) (ap + o_ + 16);                                    \
-        ra3 = *(const uint4*) (ap + o_ + 24);                                    \
-        if (q8) {                                                                \
-            rw0 = *(const uint4*) (wqp + o_);                                    \
-            rw1 = *(const uint4*) (wqp + o_ + 16);                               \
-            rs = h16_to_f(wsp[(ks) * (GK / 32)]);                                \
-        } else {                                                                 \
-            rw0 = *(const uint4*) (wbp + o_);                                    \
-            rw1 = *(const uint4*) (wbp + o_ + 8);                                \
-            rw2 = *(const uint4*) (wbp + o_ + 16);                               \
-            rw3 = *(const uint4*) (wbp + o_ + 24);                               \
-        }                                                                        \
-    }
-#define PF_GEMM_STORE(buf)                                                       \
-    {                                                                            \
-        *(uint4*) &sA[buf][sr][kh] = ra0;                                        \
-        *(uint4*) &sA[buf][sr][kh + 8] = ra1;                                    \
-        *(uint4*) &sA[buf][sr][kh + 16] = ra2;                                   \
-        *(uint4*) &sA[buf][sr][kh + 24] = ra3;                                   \
-        if (q8) q8_block_bf16(rw0, rw1, rs, rw0, rw1, rw2, rw3);                  \
-        *(uint4*) &sW[buf][sr][kh] = rw0;                                        \
-        *(uint4*) &sW[buf][sr][kh + 8] = rw1;                                    \
-        *(uint4*) &sW[buf][sr][kh + 16] = rw2;                                   \
-        *(uint4*) &sW[buf][sr][kh + 24] = rw3;                                   \
-    }
-
-    f32x16_t acc[2][2];
+    // Staging: eight lanes read a row's 128 bytes of a k step (four its 64 Q8_0 codes), so a load touches 8
+    // cache lines (16) and not 64.  Thread -> rows tid / 8 + 32 i, k 8 (tid % 8) .. +7 of A and of bf16 weights;
+    // rows tid / 4 + 64 i, k 16 (tid % 4) .. +15 of Q8_0 weights.
+    const int ar = tid >> 3, ak = (tid & 7) * 8, qr = tid >> 2, qk = (tid & 3) * 16;
+    const uint16_t* ap[NA];
+    const uint16_t* wbp[NW];
+    const int8_t* wqp[NW];
+    const uint16_t* wsp[NW];
+    auto wrow = [&](int r) {                                       // weight row of tile column r
+        const size_t n = (size_t) min(n0 + r, g.N - 1);
+        return UM ? (n & 3) * (size_t) g.um_d + (n >> 2) : n;
+    };
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NA; ++i) ap[i] = g.a + (size_t) min(m0 + ar + 32 * i, g.M - 1) * g.lda + k0 + ak;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < NW; ++i) {
+        if constexpr (Q8) {
+            wqp[i] = g.wq + wrow(qr + 64 * i) * g.K + k0 + qk;
+            wsp[i] = g.ws + wrow(qr + 64 * i) * (g.K / 32) + (k0 + qk) / 32;
+        } else {
+            wbp[i] = g.wb + wrow(ar + 32 * i) * g.K + k0 + ak;
+        }
+    }
+    // DEPTH k steps are in flight, in register sets used in turn: small launches leave a SIMD one or two waves,
+    // and a step takes as long as its loads unless they left several steps before (250 x 2,048 x 6,144 in bf16
+    // on 64-wide tiles: 37 us with two, 26 with three).  Q8_0 gains more from a fourth workgroup per CU than
+    // from a third step (the same product from Q8_0: 43 us against 56).
+    constexpr int DEPTH = SB ? 1 : Q8 ? 2 : 3;
+    u32x4_t ra[DEPTH][NA], rw[DEPTH][NW];
+    uint16_t rs[DEPTH][NW];
+    auto load = [&](int q, int ks) {                               // past the end the last step again
+        ks = min(ks, nk - 1);
+        const size_t o = (size_t) ks * GK;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) ra[q][i] = *(const u32x4_t*) (ap[i] + o);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            if constexpr (Q8) {
+                rw[q][i] = *(const u32x4_t*) (wqp[i] + o);
+                rs[q][i] = wsp[i][ks * (GK / 32)];
+            } else {
+                rw[q][i] = *(const u32x4_t*) (wbp[i] + o);
+            }
+        }
+    };
+    auto store = [&](int q, int buf) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) *(u32x4_t*) &sA[buf][ar + 32 * i][ak] = ra[q][i];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            if constexpr (Q8) {
+                const float sc = h16_to_f(rs[q][i]);
+                *(uint4*) &sW[buf][qr + 64 * i][qk] = q8_quarter_bf16(rw[q][i].x, rw[q][i].y, sc);
+                *(uint4*) &sW[buf][qr + 64 * i][qk + 8] = q8_quarter_bf16(rw[q][i].z, rw[q][i].w, sc);
+            } else {
+                *(u32x4_t*) &sW[buf][ar + 32 * i][ak] = rw[q][i];
+            }
+        }
+    };
+
+    f32x16_t acc[NB][NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-    PF_GEMM_LOAD(0);
-    PF_GEMM_STORE(0);
-    __syncthreads();
-    for (int ks = 0; ks < nk; ++ks) {
+    // step ks (in buffer ks % 2): set q held it and takes step ks + DEPTH; step ks + 1 goes to the other buffer
+    auto step = [&](int q, int ks) {
         const int buf = SB ? 0 : (ks & 1);
-        const bool more = ks + 1 < nk;
-        if (more) PF_GEMM_LOAD(ks + 1);                            // next step's loads in flight
+        load(q, ks + DEPTH);
 #pragma unroll
         for (int kk = 0; kk < GK / 16; ++kk) {
-            bf16x8_t av[2], bv[2];
+            bf16x8_t av[NB], bv[NB];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
-                av[i] = *(const bf16x8_t*) &sA[buf][wm * 64 + i * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
+            for (int i = 0; i < NB; ++i)
+                av[i] = *(const bf16x8_t*) &sA[buf][wm * (GM / 2) + i * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                bv[j] = *(const bf16x8_t*) &sW[buf][wn * 64 + j * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
+            for (int j = 0; j < NB; ++j)
+                bv[j] = *(const bf16x8_t*) &sW[buf][wn * (GN / 2) + j * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < NB; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
         }
-        if constexpr (SB) {
-            __syncthreads();                                       // every wave is done with the buffer
-            if (more) PF_GEMM_STORE(0);
-        } else {
-            if (more) PF_GEMM_STORE(buf ^ 1);
-        }
+        if constexpr (SB) __syncthreads();                         // every wave is done with the buffer
+        store((q + 1) % DEPTH, SB ? 0 : buf ^ 1);
         __syncthreads();
+    };
+#pragma unroll
+    for (int q = 0; q < DEPTH; ++q) load(q, q);
+    store(0, 0);
+    __syncthreads();
+    int ks = 0;
+    for (; ks + DEPTH <= nk; ks += DEPTH) {
+#pragma unroll
+        for (int q = 0; q < DEPTH; ++q) step(q, ks + q);
     }
-#undef PF_GEMM_LOAD
-#undef PF_GEMM_STORE
+#pragma unroll
+    for (int q = 0; q < DEPTH - 1; ++q)
+        if (ks + q < nk) step(q, ks + q);                          // workgroup-uniform
     // acc[i][j][r] = C[row 8*(r/4) + 4*(lane/32) + r%4][col lane%32] of block (i, j)
     if constexpr (UM) {
         // mixed = (sum over streams in order of xn / (1 + exp(-bf16 gate))) / 4, fp32 and bf16
@@ -190,25 +213,26 @@ __global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : 2) pf_gemm_kernel(Gem
         uint16_t (*const xs)[XS_LD] = (uint16_t (*)[XS_LD]) sAW;     // [row][stream * GN/4 + position]
 #pragma unroll
         for (int i = 0; i < GM * 4 * (GN / 4) / 8 / 256; ++i) {
-            const int pc = tid + 256 * i, rr = pc >> 4, sc = (pc >> 2) & 3, q = pc & 3;
+            constexpr int PS = GN / 32;                              // 16-byte pieces per row and stream
+            const int pc = tid + 256 * i, rr = pc / (4 * PS), sc = (pc / PS) & 3, q = pc % PS;
             const int row = min(m0 + rr, g.M - 1);
             *(uint4*) &xs[rr][sc * (GN / 4) + 8 * q] = *(const uint4*) (g.um_xn + (size_t) row * 4 * D + (size_t) sc * D + d0 + 8 * q);
         }
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < NB; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int d = (n0 + wn * 64 + j * 32 + (lane & 31)) >> 2;
+            for (int j = 0; j < NB; ++j) {
+                const int d = (n0 + wn * (GN / 2) + j * 32 + (lane & 31)) >> 2;
                 float xv[16];
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int rr = wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    const int rr = wm * (GM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     xv[r] = bf16_to_f(xs[rr][c * (GN / 4) + d - d0]);
                 }
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    const int row = m0 + wm * (GM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     const float gq = bf16_to_f(f_to_bf16(acc[i][j][r]));
                     const float term = xv[r] / (1.0f + __expf(-gq));
                     float sum = 0.f + dpp_f<0x00>(term);             // quad lanes 0..3 = streams 0..3
@@ -226,13 +250,13 @@ __global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : 2) pf_gemm_kernel(Gem
     }
     float* const y = g.y ? g.y + (size_t) ksp * g.M * g.ldy : nullptr;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = n0 + wn * 64 + j * 32 + (lane & 31);
+        for (int j = 0; j < NB; ++j) {
+            const int col = n0 + wn * (GN / 2) + j * 32 + (lane & 31);
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                const int row = m0 + wm * (GM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                 if (row < g.M && col < g.N) {
                     if (y) y[(size_t) row * g.ldy + col] = acc[i][j][r];
                     else g.yb[(size_t) row * g.ldy + col] = f_to_bf16(acc[i][j][r]);
@@ -1152,15 +1176,27 @@ int launch_pf_gemm(const PfGemm& g0, hipStream_t st) {
     }
     GemmArgs ga;
     ga.g = g;
-    ga.mt = (g.M + GM - 1) / GM;
-    ga.nt = (g.N + GN - 1) / GN;
-    WZY_REQUIRE((long long) ga.mt * ga.nt * ksplit < (1LL << 31), "pf_gemm: too many tiles");
-    const int grid = ga.mt * ga.nt * (um ? 1 : ksplit);
-    const bool sb = grid >= 512;
-    if (um && sb) hipLaunchKernelGGL((pf_gemm_kernel<true, true>), dim3(grid), dim3(256), 0, st, ga);
-    else if (um) hipLaunchKernelGGL((pf_gemm_kernel<true, false>), dim3(grid), dim3(256), 0, st, ga);
-    else if (sb) hipLaunchKernelGGL((pf_gemm_kernel<false, true>), dim3(grid), dim3(256), 0, st, ga);
-    else hipLaunchKernelGGL((pf_gemm_kernel<false, false>), dim3(grid), dim3(256), 0, st, ga);
+    auto tiles = [&](int t) { return (long long) ((g.M + t - 1) / t) * ((g.N + t - 1) / t) * ksplit; };
+    // 64 x 64 tiles where 128 x 128 ones would leave compute units idle (fewer than 256: Q8_0 250 x 2,048 x
+    // 6,144 103 -> 43 us, 1,300 x 2,048 x 2,048 43 -> 29; at 256 tiles bf16 33 us with 128, 40 with 64); from 512
+    // of the latter, one LDS buffer and more workgroups a CU.
+    const int t = tiles(128) < 256 ? 64 : 128;
+    WZY_REQUIRE(tiles(t) < (1LL << 31), "pf_gemm: too many tiles");
+    ga.mt = (g.M + t - 1) / t;
+    ga.nt = (g.N + t - 1) / t;
+    const int grid = (int) tiles(t);
+    const bool sb = t == 128 && grid >= 512, q8 = g.wq != nullptr;
+#define C_(T, U, S)                                                                                             \
+    if (q8) hipLaunchKernelGGL((pf_gemm_kernel<T, U, S, true>), dim3(grid), dim3(256), 0, st, ga);             \
+    else hipLaunchKernelGGL((pf_gemm_kernel<T, U, S, false>), dim3(grid), dim3(256), 0, st, ga)
+    if (t == 64) {
+        if (um) { C_(64, true, false); } else { C_(64, false, false); }
+    } else if (sb) {
+        if (um) { C_(128, true, true); } else { C_(128, false, true); }
+    } else {
+        if (um) { C_(128, true, false); } else { C_(128, false, false); }
+    }
+#undef C_
     WZY_LAUNCH_CHECK();
     return WZY_OK;
 }
