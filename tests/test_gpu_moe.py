@@ -255,6 +255,33 @@ def test_moe_config1_parity(wz, orc, gpu):
     assert err < 2e-3, err
 
 
+@pytest.mark.parametrize("V", [1, 15, 17, 2047, 2048, 2049, 40000, 262144])
+def test_row_top16_ties_and_specials(wz, gpu, V):
+    """Top-16 rows full of ties (small integers, so most ranks are decided by the index), with both zeros,
+    infinities and NaNs, around the 2,048-logit chunk: value descending, lower index first, NaN never
+    selected, missing entries (-inf, 2^31 - 1)."""
+    print("case top16_ties V=%d" % V, flush=True)
+    rng = np.random.default_rng(V)
+    T = 4
+    l = rng.integers(-3, 4, (T, V)).astype(np.float32)
+    l[1] = np.where(l[1] == 0, np.where(rng.random(V) < 0.5, -0.0, 0.0), -np.abs(l[1]))
+    l[2] = np.where(rng.random(V) < 0.9, -np.inf, np.nan)
+    l[3, rng.random(V) < 0.5] = np.nan
+    l[3, rng.random(V) < 0.001] = np.inf
+    ld, g, tv, ti = dev(l), DA(T, np.int32), DA(T * 16, np.float32), DA(T * 16, np.int32)
+    wz.wzy_row_top16(ld.ptr, V, T, g.ptr, tv.ptr, ti.ptr, None)
+    wz.wzy_device_sync()
+    for t in range(T):
+        ok = np.flatnonzero(~np.isnan(l[t]))
+        ids = ok[np.lexsort((ok, -l[t, ok]))][:16]
+        want_i = np.full(16, 2 ** 31 - 1, np.int64)
+        want_v = np.full(16, -np.inf, np.float32)
+        want_i[:len(ids)], want_v[:len(ids)] = ids, l[t, ids]
+        np.testing.assert_array_equal(host(ti).reshape(T, 16)[t], want_i)
+        np.testing.assert_array_equal(host(tv).reshape(T, 16)[t], want_v)
+        assert host(g)[t] == want_i[0]
+
+
 @pytest.mark.parametrize("T", [1, 2, 4, 8])
 def test_moe_reference_real_shape(wz, orc, gpu, T):
     """The reference's real MoE shape (NE 2560, NFF 640, 512 experts top-10; src/wzy_kernels_v2.cuh:8-11):

@@ -1,7 +1,7 @@
 // reduce_noalloc.hip -- allocation-free variant of the vocabulary top-16 reduction, for callers that
 // cannot call hipMalloc (code under HIP graph capture, tight serving loops, harnesses that forbid it).
 //
-// The reduction (row_topr_kernel, reduce.hip) needs a scratch of row arrival counters and per-chunk
+// The reduction (row_top16_kernel, reduce.hip) needs a scratch of row arrival counters and per-chunk
 // partial results.  Here that scratch is a file-scope device array of a fixed size, `scratch`.  Its
 // host-side name is only a stand-in for the symbol: the device address is looked up once per device
 // with hipGetSymbolAddress (each GPU holds its own copy) and only that address is ever passed to a
