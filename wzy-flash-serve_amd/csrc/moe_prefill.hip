@@ -2,7 +2,7 @@
 //
 // Launch sequence of wzy_moe_prefill (N tokens, E experts, top-K):
 //   1. pf_cvt      x fp32 -> bf16 (round to nearest even), the A operand of every GEMM
-//   2. pf_gemm     router logits [N x E] = x . router^T                      (bf16 weights)
+//   2. launch_pf_gemm  router logits [N x E] = x . router^T                  (bf16 weights)
 //   3. pf_route    per token, one wave: softmax top-K (the decode routing: probability desc, id asc,
 //                  weights renormalised by max(sum, 2^-14)) and the shared-expert gate sg = sgate . x
 //   4. pf_hist, pf_tiles, pf_scatter: entries (token, slot) grouped by expert into tiles of up to 64 or
@@ -16,7 +16,7 @@
 // pf_expert: 8 waves, 256 weight rows per workgroup, up to 128 A rows; weights staged through LDS in
 // coalesced 64-byte pieces of a row and dequantised by each lane into its v_mfma_f32_32x32x16_bf16 B fragment
 // (e2m1 x e4m3 block scale is exact in bf16, the fp32 tensor scale goes onto the accumulators;
-// Q8_0 code x fp16 scale is rounded to bf16).  pf_gemm: 64 x 64 LDS-tiled bf16 GEMM (router).
+// Q8_0 code x fp16 scale is rounded to bf16).
 // reference: pf_moe_gu_wmma_kernel, pf_moe_down_wmma_kernel, the tile builder and the shared/router
 // prefill GEMMs (src/wzy_prefill_tc.cuh:99-443), with fp16 replaced by bf16.
 #include <type_traits>
@@ -24,6 +24,7 @@
 #include "wzy_device.h"
 #include "wzy_host.h"
 #include "wzy_moe.h"
+#include "wzy_prefill.h"
 #include "wzy_route.h"
 
 using namespace wzy;
@@ -37,24 +38,12 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr int PB = 64;             // router GEMM: tile rows (M), weight rows (N) and K step
-constexpr int PB_LD = PB + 8;      // LDS row stride in bf16 (16-byte aligned rows, staggered banks)
 constexpr int PF_MAX_E = 1024;
 constexpr int EK = 64;             // expert GEMM: K step between barriers (four MFMA k16 slices)
 constexpr int EA_LD = EK + 8;      // LDS row stride of the staged activations, bf16
 
 struct PfTile {
     int e, off, cnt, pad;          // expert, first entry position, entries (at most the launch's tile size)
-};
-
-// Router GEMM logits = A . W^T over rows m0 .. m0+63 of A [a_rows x K] (bf16), bf16 weights.
-struct PfGemmArgs {
-    const uint16_t* a;
-    int a_rows, K;
-    const uint16_t* w;             // weight rows of length K
-    int n_rows;                    // weight rows
-    float* y; int y_ld;            // y[row * y_ld + n]
-    int ncb, mt;                   // 64-wide weight-row blocks and 64-row A tiles (grid = ncb * mt)
 };
 
 // Routed-expert GEMM over expert tiles.  Gate|up: A rows = x rows of the entries' tokens, output
@@ -85,83 +74,6 @@ WZY_DEV uint32_t pack_bf16(float a, float b) {
 }
 WZY_DEV float bf16_bits_to_f(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 WZY_DEV uint32_t f_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
-
-// Router GEMM tile: 64 rows x 64 weight rows, K stepped by 64 through two LDS buffers, each wave a
-// 32 x 32 block.  Workgroups go to the 8 XCDs in turn (workgroup b on XCD b % 8); when the A tile count
-// is a multiple of 8, XCD x runs the ncb weight blocks of A tiles x, x + 8, ... back to back, so each
-// A tile is fetched into one XCD's L2 once instead of once per weight block.
-__global__ void __launch_bounds__(256) pf_gemm_kernel(PfGemmArgs a) {
-    __shared__ __align__(16) uint16_t sA[2][PB][PB_LD];
-    __shared__ __align__(16) uint16_t sB[2][PB][PB_LD];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wm = w & 1, wn = w >> 1;
-    const int b = blockIdx.x;
-    int rt, cb;
-    if ((a.mt & 7) == 0) {
-        const int s = b >> 3;
-        rt = (s / a.ncb) * 8 + (b & 7);
-        cb = s % a.ncb;
-    } else {
-        rt = b / a.ncb;
-        cb = b % a.ncb;
-    }
-    const int row0 = rt * PB;
-    const int cnt = min(PB, a.a_rows - row0);
-    const int n0 = cb * PB;
-    const int sr = tid >> 2, sk = (tid & 3) * 16;                // staging: row sr, k sk .. sk+15
-    const int wrow = min(n0 + sr, a.n_rows - 1);
-    const bool a_ok = sr < cnt;
-    const uint16_t* ap = a.a + (size_t) (a_ok ? row0 + sr : 0) * a.K + sk;
-    const uint16_t* wp = a.w + (size_t) wrow * a.K + sk;
-
-    f32x16_t acc;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-    const int nk = a.K / PB;
-
-    // staging registers (scalars: an array captured by a lambda would live in scratch memory)
-    uint4 xa0 = a_ok ? *(const uint4*) ap : make_uint4(0, 0, 0, 0);
-    uint4 xa1 = a_ok ? *(const uint4*) (ap + 8) : make_uint4(0, 0, 0, 0);
-    uint4 xw0 = *(const uint4*) wp, xw1 = *(const uint4*) (wp + 8);
-    *(uint4*) &sA[0][sr][sk] = xa0;
-    *(uint4*) &sA[0][sr][sk + 8] = xa1;
-    *(uint4*) &sB[0][sr][sk] = xw0;
-    *(uint4*) &sB[0][sr][sk + 8] = xw1;
-    __syncthreads();
-    for (int ks = 0; ks < nk; ++ks) {
-        const int buf = ks & 1;
-        const bool more = ks + 1 < nk;
-        if (more) {                                              // next step's loads first
-            const size_t o = (size_t) (ks + 1) * PB;
-            xa0 = a_ok ? *(const uint4*) (ap + o) : make_uint4(0, 0, 0, 0);
-            xa1 = a_ok ? *(const uint4*) (ap + o + 8) : make_uint4(0, 0, 0, 0);
-            xw0 = *(const uint4*) (wp + o);
-            xw1 = *(const uint4*) (wp + o + 8);
-        }
-#pragma unroll
-        for (int kk = 0; kk < PB / 16; ++kk) {
-            const bf16x8_t av = *(const bf16x8_t*) &sA[buf][wm * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
-            const bf16x8_t bv = *(const bf16x8_t*) &sB[buf][wn * 32 + (lane & 31)][kk * 16 + (lane >> 5) * 8];
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
-        }
-        if (more) {
-            *(uint4*) &sA[buf ^ 1][sr][sk] = xa0;
-            *(uint4*) &sA[buf ^ 1][sr][sk + 8] = xa1;
-            *(uint4*) &sB[buf ^ 1][sr][sk] = xw0;
-            *(uint4*) &sB[buf ^ 1][sr][sk + 8] = xw1;
-        }
-        __syncthreads();
-    }
-
-    // acc[i] = C[row 8*(i/4) + 4*(lane/32) + i%4][col lane%32] of the wave's block
-    const int col = wn * 32 + (lane & 31);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int m = wm * 32 + 8 * (i / 4) + 4 * (lane >> 5) + (i & 3);
-        const int n = n0 + col;
-        if (m < cnt && n < a.n_rows) a.y[(size_t) (row0 + m) * a.y_ld + n] = acc[i];
-    }
-}
 
 // MFMA B fragment (8 consecutive k of one weight row) from one 16-value NVFP4 sub-block: bytes
 // w0 (0..3), w1 (4..7), byte i = value i (low nibble) | value i+8 (high nibble).  The lane half
@@ -515,7 +427,15 @@ __global__ void __launch_bounds__(256) pf_route_kernel(const float* __restrict__
         p[i] = idx < E ? v : -INFINITY;
     }
     float s = 0.f;
-    for (int d = lane; d < D; d += 64) s = fmaf(bf16_bits_to_f(sgate[d]), bf16_bits_to_f(xb[(size_t) t * D + d]), s);
+    for (int d = lane * 8; d < D; d += 512) {                    // D a multiple of 256: whole 16-byte pieces
+        const uint4 gv = *(const uint4*) (sgate + d), xv = *(const uint4*) (xb + (size_t) t * D + d);
+        const uint32_t ga[4] = {gv.x, gv.y, gv.z, gv.w}, xa[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            s = fmaf(bf16_lo(ga[i]), bf16_lo(xa[i]), s);
+            s = fmaf(bf16_hi(ga[i]), bf16_hi(xa[i]), s);
+        }
+    }
     s = wave_sum(s);
     if (lane == 0) sg[t] = s;
     int my_id;
@@ -716,19 +636,18 @@ int pf_check(const wzy_moe_weights* w, int N) {
     WZY_REQUIRE(E >= 1 && E <= PF_MAX_E && E % 64 == 0, "wzy_moe_prefill: n_exp must be a multiple of 64 up to %d",
                 PF_MAX_E);
     WZY_REQUIRE(K >= 1 && K <= MOE_MAX_K && K <= E, "wzy_moe_prefill: top_k must be in [1, %d]", MOE_MAX_K);
-    WZY_REQUIRE((int64_t) (E / PB) * ((N + PB - 1) / PB) * 256 <= INT32_MAX && (int64_t) N * D <= INT32_MAX,
+    WZY_REQUIRE((int64_t) (E / 64) * ((N + 63) / 64) * 256 <= INT32_MAX && (int64_t) N * D <= INT32_MAX,
                 "wzy_moe_prefill: n_tok x n_embd exceeds the launch grids");
     return WZY_OK;
 }
 
 // The launch sequence; with `ev`, event i is recorded before launch group i and event PF_N_STAGES
 // after the last one.
-void pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, const PfWs& ws, hipStream_t st,
+int pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, const PfWs& ws, hipStream_t st,
                 hipEvent_t* ev) {
     const int D = w->n_embd, F = w->n_ff, E = w->n_exp, K = w->top_k;
     const int n_ent = N * K;
     const MoeOffsets o = moe_offsets(D, F);
-    const int mt = (N + PB - 1) / PB;
     auto mark = [&](int i) {
         if (ev) (void) hipEventRecord(ev[i], st);
     };
@@ -737,13 +656,10 @@ void pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, co
     hipLaunchKernelGGL(pf_cvt_kernel, dim3((unsigned) ((nx / 4 + 255) / 256)), dim3(256), 0, st, x, ws.xb, nx,
                        ws.cursor, E);
     mark(1);
-    {   // router logits
-        PfGemmArgs a{};
-        a.a = ws.xb; a.a_rows = N; a.K = D;
-        a.w = w->router; a.n_rows = E;
-        a.y = ws.logits; a.y_ld = E;
-        a.ncb = E / PB; a.mt = mt;
-        hipLaunchKernelGGL(pf_gemm_kernel, dim3((unsigned) (a.ncb * mt)), dim3(256), 0, st, a);
+    {   // router logits, on the dense projections' kernel
+        PfGemm g{};
+        g.a = ws.xb; g.lda = D; g.M = N; g.N = E; g.K = D; g.wb = w->router; g.y = ws.logits; g.ldy = E;
+        WZY_TRY(launch_pf_gemm(g, st));
     }
     mark(2);
     if (E <= 512)
@@ -800,6 +716,7 @@ void pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, co
             hipLaunchKernelGGL((pf_combine_kernel<8, false>), cg, dim3(256), 0, st, ws.y, ws.ent_pos, ws.wts, K, D, comb);
     }
     mark(8);
+    return WZY_OK;
 }
 
 PfWs pf_ws_for(const wzy_moe_weights* w, int N, void* workspace, size_t workspace_bytes) {
@@ -818,7 +735,7 @@ extern "C" int wzy_moe_prefill(const wzy_moe_weights* w, const float* x, int n_t
                 "wzy_moe_prefill: workspace too small");
     hipStream_t st = as_stream(stream);
     const PfWs ws = pf_ws_for(w, N, workspace, workspace_bytes);
-    pf_enqueue(w, x, N, comb, ws, st, nullptr);
+    WZY_TRY(pf_enqueue(w, x, N, comb, ws, st, nullptr));
     if (ids) WZY_HIP_TRY(hipMemcpyAsync(ids, ws.ids, (size_t) N * K * sizeof(int), hipMemcpyDeviceToDevice, st));
     if (wts) WZY_HIP_TRY(hipMemcpyAsync(wts, ws.wts, (size_t) N * K * sizeof(float), hipMemcpyDeviceToDevice, st));
     WZY_LAUNCH_CHECK();
@@ -837,9 +754,10 @@ extern "C" int wzy_moe_prefill_time(const wzy_moe_weights* w, const float* x, in
     for (int i = 0; i <= PF_N_STAGES; ++i) WZY_HIP_TRY(hipEventCreate(&ev[i]));
     double acc[PF_N_STAGES] = {};
     int rc = WZY_OK;
-    pf_enqueue(w, x, n_tok, comb, ws, st, nullptr);                 // warm-up
+    rc = pf_enqueue(w, x, n_tok, comb, ws, st, nullptr);            // warm-up
     for (int it = 0; it < iters && rc == WZY_OK; ++it) {
-        pf_enqueue(w, x, n_tok, comb, ws, st, ev);
+        rc = pf_enqueue(w, x, n_tok, comb, ws, st, ev);
+        if (rc != WZY_OK) break;
         if (hipEventSynchronize(ev[PF_N_STAGES]) != hipSuccess) { rc = WZY_EHIP; break; }
         for (int i = 0; i < PF_N_STAGES; ++i) {
             float ms = 0.f;
