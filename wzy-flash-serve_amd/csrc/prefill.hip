@@ -709,31 +709,34 @@ __global__ void __launch_bounds__(128) pf_gdn_norm_kernel(PfGdn g) {
 // ---------------------------------------------------------------------------------------------
 // QSA
 // ---------------------------------------------------------------------------------------------
-constexpr int PR_ROWS = 4;                    // rows per prep workgroup
-
-// grid (qh + kvh + ih, ceil(B / PR_ROWS)), 256 threads: q heads, kv heads (+ INT8 append), indexer q heads
+// One wave per (row, head): q heads, kv heads (+ INT8 append), indexer q heads.  Bound by reading and writing
+// the heads once (8,192 rows: 0.45 GB); with a workgroup per head and two barriers in each norm the loads of a
+// head waited for the one before it (8,191 rows 265 -> 108 us, 1,300 rows 40 -> 24 us; 4.2 TB/s).
 __global__ void __launch_bounds__(256) pf_qsa_prep_kernel(PfQsaPrep a, int B) {
-    __shared__ float s_vals[256];
-    __shared__ float s_red[4];
+    __shared__ float s_rot[4][128];
     const QsaDims& dm = a.dm;
-    const int role = blockIdx.x, tid = threadIdx.x;
-    const int base = *a.pos, hd = dm.hd, kvd = dm.kvh * dm.hd;
-    for (int t = blockIdx.y * PR_ROWS; t < min(B, (int) (blockIdx.y + 1) * PR_ROWS); ++t) {
-        const int pos = base + t;
-        if (role < dm.qh) {
-            norm_rope(a.qg + (size_t) t * dm.qh * 2 * hd + (size_t) role * 2 * hd, hd, a.q_norm, a.cos_tab, a.sin_tab, pos,
-                      dm.n_rot, dm.eps, s_vals, s_red);
-        } else if (role < dm.qh + dm.kvh) {
-            const int j = role - dm.qh;
-            float* kp = a.kk + (size_t) t * kvd + (size_t) j * hd;
-            norm_rope(kp, hd, a.k_norm, a.cos_tab, a.sin_tab, pos, dm.n_rot, dm.eps, s_vals, s_red);
-            if (tid < hd) qsa_kv_store(dm, a.kv, pos, j, kp[tid], a.vv[(size_t) t * kvd + (size_t) j * hd + tid]);
-            __syncthreads();
-        } else {
-            const int i = role - dm.qh - dm.kvh;
-            norm_rope(a.q_idx + (size_t) t * dm.ih * dm.idim + (size_t) i * dm.idim, dm.idim, a.iq_norm, a.cos_tab,
-                      a.sin_tab, pos, dm.n_rot, dm.eps, s_vals, s_red);
-        }
+    const int lane = threadIdx.x & 63, roles = dm.qh + dm.kvh + dm.ih;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * 4 + w, t = i / roles, role = i % roles;
+    if (t >= B) return;                          // wave-uniform; no barrier follows
+    const int pos = *a.pos + t, hd = dm.hd, kvd = dm.kvh * dm.hd;
+    float y[4];
+    if (role < dm.qh) {
+        norm_rope_wave(a.qg + (size_t) t * dm.qh * 2 * hd + (size_t) role * 2 * hd, hd, a.q_norm, a.cos_tab, a.sin_tab, pos,
+                       dm.n_rot, dm.eps, s_rot[w], y);
+    } else if (role < dm.qh + dm.kvh) {
+        const int j = role - dm.qh;
+        const size_t at = (size_t) t * kvd + (size_t) j * hd;
+        float v[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) v[g] = a.vv[at + 64 * g + lane];
+        norm_rope_wave(a.kk + at, hd, a.k_norm, a.cos_tab, a.sin_tab, pos, dm.n_rot, dm.eps, s_rot[w], y);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) qsa_kv_store_group(dm, a.kv, pos, j, g, y[g], v[g]);
+    } else {
+        const int h = role - dm.qh - dm.kvh;
+        norm_rope_wave(a.q_idx + (size_t) t * dm.ih * dm.idim + (size_t) h * dm.idim, dm.idim, a.iq_norm, a.cos_tab,
+                       a.sin_tab, pos, dm.n_rot, dm.eps, s_rot[w], y);
     }
 }
 
@@ -1250,7 +1253,7 @@ int launch_pf_gdn(const PfGdn& g, hipStream_t st) {
 int launch_pf_qsa_prep(const PfQsaPrep& a, int B, hipStream_t st) {
     WZY_TRY(qsa_check_dims(a.dm));
     const int roles = a.dm.qh + a.dm.kvh + a.dm.ih;
-    hipLaunchKernelGGL(pf_qsa_prep_kernel, dim3(roles, (B + PR_ROWS - 1) / PR_ROWS), dim3(256), 0, st, a, B);
+    hipLaunchKernelGGL(pf_qsa_prep_kernel, dim3((unsigned) (((int64_t) roles * B + 3) / 4)), dim3(256), 0, st, a, B);
     WZY_LAUNCH_CHECK();
     return WZY_OK;
 }

@@ -31,12 +31,55 @@ WZY_DEV void norm_rope(float* p, int hd, const float* gamma, const float* cos_ta
     __syncthreads();
 }
 
-// Per-64 INT8 quantisation of element `threadIdx.x` (< hd) of KV head j's k and v rows into the
-// store slot of position pos: scale = fp16(max|x| / 127) per 64-element group (one wave per group,
-// every lane of the wave active), code = clamp(round(x / scale), +-127).
-// reference: kv_append_int8_multi (src/wzy_qsa_256k.cuh:86-143)
-WZY_DEV void qsa_kv_store(const QsaDims& dm, const QsaKv& kv, int pos, int j, float kval, float vval) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// RMSNorm + RoPE of one head vector p[0..hd) in place by one wave: lane l owns elements l + 64 j and returns
+// them in y.  Same values as norm_rope (its sum adds the 64-element groups' sums in order); no barrier, and
+// every load is issued before the reduction.  n_rot <= 128; s_rot: 128 floats of the wave's own.
+WZY_DEV void norm_rope_wave(float* p, int hd, const float* gamma, const float* cos_tab, const float* sin_tab, int pos,
+                            int n_rot, float eps, float* s_rot, float (&y)[4]) {
+    const int lane = threadIdx.x & 63, half = n_rot / 2;
+    float x[4], g[4], c[2] = {0.f, 0.f}, s[2] = {0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int i = lane + 64 * j;
+        x[j] = i < hd ? p[i] : 0.f;
+        g[j] = i < hd ? gamma[i] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        if (lane + 64 * j < n_rot) {
+            const size_t at = (size_t) pos * half + (lane + 64 * j) % half;
+            c[j] = cos_tab[at];
+            s[j] = sin_tab[at];
+        }
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ss += wave_sum(x[j] * x[j]);
+    const float sc = 1.0f / sqrtf(ss / (float) hd + eps);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) y[j] = x[j] * (sc * g[j]);
+    s_rot[lane] = y[0];
+    s_rot[lane + 64] = y[1];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int i = lane + 64 * j;
+        if (i < n_rot) {
+            const int pr = i % half;
+            const float a = s_rot[pr], d = s_rot[pr + half];
+            y[j] = (i < half) ? (a * c[j] - d * s[j]) : (a * s[j] + d * c[j]);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (lane + 64 * j < hd) p[lane + 64 * j] = y[j];
+}
+
+// Per-64 INT8 quantisation of group g of KV head j's k and v rows (lane = element, every lane of the wave
+// active) into the store slot of position pos: scale = fp16(max|x| / 127), code = clamp(round(x / scale),
+// +-127).  reference: kv_append_int8_multi (src/wzy_qsa_256k.cuh:86-143)
+WZY_DEV void qsa_kv_store_group(const QsaDims& dm, const QsaKv& kv, int pos, int j, int g, float kval, float vval) {
+    const int lane = threadIdx.x & 63;
     const int hd = dm.hd, kvd = dm.kvh * dm.hd;
     const float kmax = wave_max(fabsf(kval)), vmax = wave_max(fabsf(vval));
     const uint16_t kh = f_to_h16(kmax / 127.0f), vh = f_to_h16(vmax / 127.0f);
@@ -44,12 +87,18 @@ WZY_DEV void qsa_kv_store(const QsaDims& dm, const QsaKv& kv, int pos, int j, fl
     const int kqi = kdq > 0.f ? max(-127, min(127, rn_int(kval / kdq))) : 0;
     const int vqi = vdq > 0.f ? max(-127, min(127, rn_int(vval / vdq))) : 0;
     const size_t slot = qsa_kv_slot(pos, dm);
-    kv.kq[slot * kvd + (size_t) j * hd + tid] = (int8_t) kqi;
-    kv.vq[slot * kvd + (size_t) j * hd + tid] = (int8_t) vqi;
+    const int i = g * 64 + lane;
+    kv.kq[slot * kvd + (size_t) j * hd + i] = (int8_t) kqi;
+    kv.vq[slot * kvd + (size_t) j * hd + i] = (int8_t) vqi;
     if (lane == 0) {
-        kv.ks[slot * (kvd / 64) + (size_t) j * (hd / 64) + w] = kh;
-        kv.vs[slot * (kvd / 64) + (size_t) j * (hd / 64) + w] = vh;
+        kv.ks[slot * (kvd / 64) + (size_t) j * (hd / 64) + g] = kh;
+        kv.vs[slot * (kvd / 64) + (size_t) j * (hd / 64) + g] = vh;
     }
+}
+
+// all groups of a head by one workgroup: element `threadIdx.x` (< hd), one wave per group
+WZY_DEV void qsa_kv_store(const QsaDims& dm, const QsaKv& kv, int pos, int j, float kval, float vval) {
+    qsa_kv_store_group(dm, kv, pos, j, threadIdx.x >> 6, kval, vval);
 }
 
 // Indexer key of one block (threads d < idim; 256 threads): the mean of the block's iblk cells,
