@@ -637,6 +637,35 @@ def check_chunk_sampled(wz, orc, st, om, cfg, p0, toks, rows, label):
     floor_summary(fo, 1e-3)
 
 
+@pytest.mark.parametrize("n_ctx,B", [(14500, 2048), (29003, 1801)])
+def test_prefill_block_scores_do_not_depend_on_the_launch(wz, gpu, n_ctx, B):
+    """Long contexts give a scoring workgroup several groups of 256 blocks (two of 17, three of 31 here: a last
+    workgroup with fewer), short launches one.  The scores of a chunk in one launch equal those of its parts."""
+    print("case block_scores %d %d" % (n_ctx, B), flush=True)
+    cfg = baseline_cfg(1, n_ctx + B + 8, qsa_period=1)
+    toks = [int(t) for t in np.random.default_rng(6).integers(0, cfg.n_vocab, B)]
+
+    def scores(parts):
+        st = wzy_amd.Stage(cfg)
+        try:
+            st.load_synthetic(SEED, n_ctx)
+            wz.wzy_stage_set_trace(st.h, 1)
+            out, at = [], 0
+            for n in parts:
+                st.prefill(n_ctx + at, toks[at:at + n])
+                st.sync()
+                g = st.read(-1, "trace.pf_scores", np.float32).reshape(-1, cfg.ctx_max // 4 + 2)
+                out += [g[t, :(n_ctx + at + t + 1) // 4 + 1].copy() for t in range(n)]
+                at += n
+            return out
+        finally:
+            st.close()
+
+    whole = scores([B])
+    for t, (x, y) in enumerate(zip(whole, scores([700, 333, B - 1033]))):
+        assert np.isfinite(x).all() and np.array_equal(x, y), t
+
+
 @pytest.mark.timeout(900)
 def test_prefill_8192_rows_baseline_shapes(wz, orc, gpu):
     """The bench's chunk length, 8,192 rows, through four BASELINE-shape layers (GDN, GDN, GDN, QSA)

@@ -20,6 +20,7 @@
 //                matrix operands).
 // reference: PrefillStageCtx::run_stage_prefill and its kernels (src/wzy_prefill_tc.cuh:20-98,
 // 546-1058; src/wzy_qsa_wmma.cuh:5-489), with cuBLAS fp16 GEMMs replaced by bf16 MFMA GEMMs.
+#include <algorithm>
 #include <type_traits>
 
 #include "wzy_device.h"
@@ -798,16 +799,18 @@ __global__ void __launch_bounds__(128) pf_idx_tail_kernel(PfIdxAppend a, int p0,
 
 // Indexer block scores of the chunk's rows on MFMA: score[t][b] = sum over heads h of
 // relu(q_h[t] . key[b]), fp16 queries and keys with fp32 products and sums (v_mfma_f32_32x32x16_f16,
-// as the reference's prefill scorer runs on WMMA).  Workgroup = 32 rows x 256 blocks, wave w: blocks
-// 64w .. 64w+63 as two 32 x 32 tiles, the four heads' accumulators side by side; the queries are
-// staged in LDS as fp16, each wave loads its keys' k slices straight into B fragments.  Only complete
+// as the reference's prefill scorer runs on WMMA).  Workgroup = 32 rows x `groups` x 256 blocks, wave w:
+// blocks 64w .. 64w+63 of a group as two 32 x 32 tiles, the four heads' accumulators side by side; the queries
+// are staged in LDS as fp16, each wave loads its keys' k slices straight into B fragments, one tile ahead.  With
+// one group a workgroup staged 64 KB of queries for two tiles a wave and no load was in flight while a tile was
+// multiplied (2,048 rows at 33-41 thousand cells 96 -> 53 us, 1,300 at 9-10 thousand 39 -> 23, the open block below included).  Only complete
 // blocks of rows whose context exceeds top_k are written; the row group's first workgroup also
 // scores the open block against the placeholder key (fp32, +1e9 while the block is partial), as the
 // decode scorer does.  (qsa_block_scores_wmma, src/wzy_qsa_wmma.cuh:492-612)
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 constexpr int PS_ROWS = 32, PS_BLOCKS = 256;
 
-__global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
+__global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a, int groups) {
     __shared__ __align__(16) _Float16 sQ[4][PS_ROWS][128 + 8];
     const QsaDims& dm = a.dm;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -816,7 +819,7 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
     const int B = dm.iblk, IH = dm.ih;
     const int n_kv_max = base + nrows;
     if (n_kv_max <= dm.topk) return;                 // short context: identity selection
-    const int b0 = blockIdx.x * PS_BLOCKS;
+    const int b0 = blockIdx.x * groups * PS_BLOCKS;
     const bool tail_wg = blockIdx.x == 0;
     const int b_lim = min(a.max_b, n_kv_max / B);
     if (b0 >= b_lim && !tail_wg) return;
@@ -835,18 +838,21 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
     if (b0 + 64 * w < b_lim) {
         // one 32-block tile at a time: 64 accumulator registers, so several workgroups share a CU
         const int kb = (lane >> 5) * 8;
+        const auto block = [&](int c) { return b0 + (c >> 1) * PS_BLOCKS + 64 * w + 32 * (c & 1) + (lane & 31); };
+        const auto key = [&](int c) {                // past the end: the last row again
+            return (const _Float16*) a.pooled + (size_t) min(block(c), b_lim - 1) * 128 + kb;
+        };
+        f16x8_t bv[8];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int b = b0 + 64 * w + 32 * c + (lane & 31);
-            const _Float16* kp = (const _Float16*) a.pooled + (size_t) min(b, b_lim - 1) * 128 + kb;
+        for (int ks = 0; ks < 8; ++ks) bv[ks] = *(const f16x8_t*) (key(0) + 16 * ks);
+        for (int c = 0; c < 2 * groups && block(c) - (lane & 31) < b_lim; ++c) {      // wave-uniform
+            const int b = block(c);
+            const _Float16* kn = key(c + 1);
             f32x16_t acc[4];
 #pragma unroll
             for (int h = 0; h < 4; ++h)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[h][i] = 0.f;
-            f16x8_t bv[8];
-#pragma unroll
-            for (int ks = 0; ks < 8; ++ks) bv[ks] = *(const f16x8_t*) (kp + 16 * ks);
 #pragma unroll
             for (int ks = 0; ks < 8; ++ks) {
 #pragma unroll
@@ -855,8 +861,11 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
                     const f16x8_t av = *(const f16x8_t*) &sQ[h][lane & 31][16 * ks + kb];
                     acc[h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv[ks], acc[h], 0, 0, 0);
                 }
+                bv[ks] = *(const f16x8_t*) (kn + 16 * ks);           // the next tile's
             }
-            // acc[h][i] = q_h[row 8*(i/4) + 4*(lane/32) + i%4] . key[block 32c + lane%32]
+            // acc[h][i] = q_h[row 8*(i/4) + 4*(lane/32) + i%4] . key[block b, lane%32 of the tile]; the block is
+            // complete for rows with n_kv >= (b + 1) B (no division per row)
+            const int t_min = max((b + 1) * B, dm.topk + 1) - base - 1;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int t = 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
@@ -864,26 +873,38 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a) {
 #pragma unroll
                 for (int h = 0; h < 4; ++h)
                     if (h < IH) sc += acc[h][i] > 0.f ? acc[h][i] : 0.f;
-                const int n_kv = base + t + 1;
-                if (t < nrows && n_kv > dm.topk && b < n_kv / B) scores[(size_t) t * a.max_b + b] = sc;
+                if (t >= t_min && t < nrows) scores[(size_t) t * a.max_b + b] = sc;
             }
         }
     }
-    // open block: fp32 dot with the placeholder key (wave w handles rows w, w + 4, ...)
+    // open block: fp32 dot with the placeholder key (wave w handles rows w, w + 4, ...), four rows' loads at a
+    // time (a load per row and head, each waited for, kept this workgroup busy after all others had ended)
     if (tail_wg) {
-        for (int t = w; t < nrows; t += 4) {
-            const int n_kv = base + t + 1;
-            const int nbid = n_kv / B;
-            if (n_kv <= dm.topk || nbid >= a.max_b) continue;
-            float score = 0.f;
-            for (int h = 0; h < IH; ++h) {
-                float p = 0.f;
-                for (int k = lane; k < 128; k += 64) p = fmaf(a.dead[k], q_idx[(size_t) t * IH * 128 + (size_t) h * 128 + k], p);
-                p = wave_sum(p);
-                score += p > 0.f ? p : 0.f;
+        constexpr int TR = 4;
+        const float d0 = a.dead[lane], d1 = a.dead[lane + 64];
+        const float* qi = IH > 0 ? q_idx : a.dead;   // without heads any readable row: nothing of it is used
+        for (int t0 = w; t0 < nrows; t0 += 4 * TR) {
+            float q[TR][4][2];
+#pragma unroll
+            for (int r = 0; r < TR; ++r)
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const float* qp = qi + ((size_t) min(t0 + 4 * r, nrows - 1) * IH + max(0, min(h, IH - 1))) * 128 + lane;
+                    q[r][h][0] = qp[0];
+                    q[r][h][1] = qp[64];
+                }
+#pragma unroll
+            for (int r = 0; r < TR; ++r) {
+                const int t = t0 + 4 * r, n_kv = base + t + 1, nbid = n_kv / B;
+                float score = 0.f;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const float p = wave_sum(fmaf(d1, q[r][h][1], fmaf(d0, q[r][h][0], 0.f)));
+                    if (h < IH) score += p > 0.f ? p : 0.f;
+                }
+                if (n_kv % B != 0) score += 1e9f;
+                if (lane == 0 && t < nrows && n_kv > dm.topk && nbid < a.max_b) scores[(size_t) t * a.max_b + nbid] = score;
             }
-            if (n_kv % B != 0) score += 1e9f;
-            if (lane == 0) scores[(size_t) t * a.max_b + nbid] = score;
         }
     }
 }
@@ -1273,14 +1294,18 @@ int launch_pf_idx_append(const PfIdxAppend& a, int p0, int B, hipStream_t st) {
     return WZY_OK;
 }
 
-int launch_pf_scores(const QsaScoreArgs& a0, int rows, hipStream_t st) {
+int launch_pf_scores(const QsaScoreArgs& a0, int rows, int max_n_kv, hipStream_t st) {
     WZY_TRY(qsa_check_dims(a0.dm));
     WZY_REQUIRE(a0.dm.idim == 128 && a0.dm.ih <= 4, "pf_scores: indexer layout unsupported");
     WZY_REQUIRE(rows >= 1 && (rows + PS_ROWS - 1) / PS_ROWS <= 65535, "pf_scores: %d rows", rows);
     QsaScoreArgs a = a0;
     a.rows = rows;
-    const dim3 grid((a.max_b + PS_BLOCKS - 1) / PS_BLOCKS, (rows + PS_ROWS - 1) / PS_ROWS);
-    hipLaunchKernelGGL(pf_score_kernel, grid, dim3(256), 0, st, a);
+    // Groups of 256 blocks per workgroup: as many as leave about two workgroups a CU.  Column 0 also takes the
+    // open blocks, so there is always one.
+    const int rg = (rows + PS_ROWS - 1) / PS_ROWS;
+    const int bg = std::max(1, (std::min(a.max_b, max_n_kv / a.dm.iblk) + PS_BLOCKS - 1) / PS_BLOCKS);
+    const int groups = (int) std::max<int64_t>(1, (int64_t) rg * bg / 512);
+    hipLaunchKernelGGL(pf_score_kernel, dim3((bg + groups - 1) / groups, rg), dim3(256), 0, st, a, groups);
     WZY_LAUNCH_CHECK();
     return WZY_OK;
 }
