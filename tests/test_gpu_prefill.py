@@ -396,6 +396,26 @@ def test_stage_prefill_at_recurrence_buffer_edges(wz, orc, gpu, p0, B, prefix):
     test_stage_prefill_matches_oracle(wz, orc, gpu, p0, B, prefix)
 
 
+def test_stage_prefill_at_attention_chunk_edges(wz, orc, gpu):
+    """Rows that attend 1 to 300 cells, every one of them: each of the four waves of an attention workgroup takes
+    no chunk of 32 cells, one, two or three, whole or cut (edges at 32, 128, 256 and 288 cells)."""
+    print("case prefill_attention_chunk_edges", flush=True)
+    cfg = pf_cfg(n_layers=2, topk=512)
+    cfg.qsa_period = 1
+    B = 300
+    toks = [int(t) for t in np.random.default_rng(17).integers(0, cfg.n_vocab, B)]
+    st = wzy_amd.Stage(cfg)
+    try:
+        st.load_synthetic(SEED, 0)
+        wz.wzy_stage_set_trace(st.h, 1)
+        om = OracleModel(wz, st, cfg, SEED)
+        st.prefill(0, toks)
+        st.sync()
+        check_chunk(wz, orc, st, om, cfg, 0, toks, "attention chunk edges")
+    finally:
+        st.close()
+
+
 def run_chunks(cfg, toks, splits, seed=SEED, n_ctx=0):
     st = wzy_amd.Stage(cfg)
     st.load_synthetic(seed, n_ctx)

@@ -1031,6 +1031,7 @@ __global__ void __launch_bounds__(256, 2) pf_attn_kernel(PfAttn a) {
     if (w < nch) {
         rid = read_id(w);
         if (lane < AT_C) sOff[w][0][lane] = rid;
+        wave_lds_sync();
         rid = read_id(w + 4);
         AT_LOAD_K(0)
         AT_LOAD_V(0)
@@ -1038,6 +1039,7 @@ __global__ void __launch_bounds__(256, 2) pf_attn_kernel(PfAttn a) {
     for (int c = w, it = 0; c < nch; c += 4, ++it) {
         const int nx = (it + 1) & 1;
         if (lane < AT_C) sOff[w][nx][lane] = rid;
+        wave_lds_sync();
         rid = read_id(c + 8);
         // S^T of the chunk's two 16-cell tiles
         f32x4_t sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};

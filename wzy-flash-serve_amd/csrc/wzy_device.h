@@ -32,6 +32,15 @@ WZY_DEV int rn_int(float x) { return (int) __builtin_rintf(x); }
 WZY_DEV float sigmoidf_(float x) { return 1.0f / (1.0f + __expf(-x)); }
 WZY_DEV float siluf_(float x) { return x / (1.0f + __expf(-x)); }
 
+// Between a wave's stores to LDS that only it uses and the loads of them by other lanes: LDS runs a wave's
+// accesses in order, so no instruction is needed, but without this the compiler may move a load above a store
+// that it proves different for the same lane.
+WZY_DEV void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------------------------
 // DPP / swizzle wave reductions (64 lanes)
 // ---------------------------------------------------------------------------------------------

@@ -59,8 +59,7 @@ WZY_DEV void norm_rope_wave(float* p, int hd, const float* gamma, const float* c
     for (int j = 0; j < 4; ++j) y[j] = x[j] * (sc * g[j]);
     s_rot[lane] = y[0];
     s_rot[lane + 64] = y[1];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int i = lane + 64 * j;
