@@ -416,6 +416,56 @@ def test_stage_prefill_at_attention_chunk_edges(wz, orc, gpu):
         st.close()
 
 
+class QsaDims(C.Structure):                       # csrc/wzy_qsa.h
+    _fields_ = [(n, C.c_int) for n in ("qh", "kvh", "hd", "n_rot", "ih", "idim", "iblk", "topk", "ctx_max", "ring_cap",
+                                       "sinks")] + [("eps", C.c_float), ("window", C.c_int), ("f16_above", C.c_int)]
+
+
+class PfAttn(C.Structure):                        # csrc/wzy_prefill.h
+    _fields_ = [("dm", QsaDims)] + [(n, C.c_void_p) for n in ("pos", "qg", "kq", "ks", "vq", "vs", "sel", "out")]
+
+
+def test_attention_weights_keep_the_largest_exact(wz, gpu):
+    """A softmax weight of 1 is exact in fp16, so the largest one adds no rounding of its own.  One wave sees a
+    cell of weight 2^-3.6 to 2^-5.9 in its first chunk (with V = 0) and the largest in its second; every other
+    cell's weight underflows to zero.  The output is then v / (1 + 2^-z) up to fp32 rounding (below 2^-20), so its
+    bf16 bits are known wherever that is not within 2^-19 of a rounding tie.  Weights against the first chunk's
+    maximum would be 12 to 60, rounded by up to 2^-11: one element in forty falls the other way."""
+    print("case attention_largest_weight", flush=True)
+    heads, hd, n_kv, lo, hi = 12, 256, 256, 5, 130
+    rng = np.random.default_rng(3)
+    s = (2.5 + np.arange(heads) * 0.125 + 0.0078125).astype(np.float32)            # fp16 numbers
+    qg = np.zeros((heads, 2, hd), np.float32)
+    qg[:, 0, 0] = 16 * s                                                           # the kernel divides by 16
+    qg[:, 1] = 100.0                                                               # sigmoid 1 in fp32
+    kq = np.zeros((n_kv, hd), np.int8)
+    kq[:, 0] = -127
+    kq[[lo, hi], 0] = 64
+    ks = np.ones((n_kv, hd // 64), np.float16)
+    ks[lo], ks[hi] = 1 / 64, 1 / 32                                                # scores s and 2 s
+    vq = rng.integers(1, 128, (n_kv, hd)).astype(np.int8)
+    vq[lo] = 0
+    vs = rng.uniform(2.0 ** -7, 2.0 ** -6, (n_kv, hd // 64)).astype(np.float16)
+    dims = QsaDims(heads, 1, hd, 64, 4, 128, 4, 2048, n_kv, 0, 0, 1e-6, 0, 0)
+    d = [DA.from_numpy(np.ascontiguousarray(x).ravel()) for x in
+         (np.array([n_kv - 1], np.int32), qg, kq, ks.view(np.uint16), vq, vs.view(np.uint16),
+          np.arange(2048, dtype=np.int32))]
+    out = DA(heads * hd, np.uint16)
+    arg = PfAttn(dims, *[x.ptr for x in d], out.ptr)
+    # internal to the library: no entry point takes a query as it stands
+    launch = C.CDLL(wz.path)["_ZN3wzy14launch_pf_attnERKNS_6PfAttnEiP12ihipStream_t"]
+    assert launch(C.byref(arg), 1, None) == 0
+    wz.wzy_device_sync()
+    v = (vq[hi].astype(np.float16) * np.repeat(vs[hi], 64)).astype(np.float64)
+    want = v[None, :] / (1.0 + np.exp(-s.astype(np.float64)))[:, None]
+    low = bits_to_f32((want.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)).astype(np.float64)
+    tie = low + 2.0 ** (np.floor(np.log2(want)) - 8)                               # halfway to the next bf16
+    sure = np.abs(want - tie) > want * 2.0 ** -19
+    assert sure.mean() > 0.99
+    got = out.numpy().reshape(heads, hd)
+    np.testing.assert_array_equal(got[sure], bf16_bits(want)[sure])
+
+
 def run_chunks(cfg, toks, splits, seed=SEED, n_ctx=0):
     st = wzy_amd.Stage(cfg)
     st.load_synthetic(seed, n_ctx)

@@ -922,8 +922,11 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a, int gr
 //                 the same eight cells, regrouped from cells x dims to dims x cells by byte permutes.
 // Codes become fp16 exactly as 1024 + (code + 128) - 1152 (a byte under the exponent of 1024), then
 // code * scale is rounded to fp16 once, two at a time, as a product of fp16 numbers.
-// The softmax keeps a reference exponent per head that a chunk's maximum moves only when it exceeds it by
-// more than 2^AT_LAZY (fp16 weights up to 64 lose nothing), so most chunks rescale no accumulator.
+// The softmax's reference exponent is the running maximum of the wave's chunks, so the largest weight is 1
+// and the weights beside it are rounded to fp16 at the top of its binades: their share of the error against
+// 64 bits is 1.5e-4 at scores of spread 1 and 0.65e-4 at spread 2.  (A reference moved only past a factor of
+// 2^6 rescales fewer accumulators and has 2.1e-4 and 1.4e-4; one running maximum for all cells, as in the kernel
+// before this one, 1.7e-4 and 0.88e-4.  8,192 rows take the same time either way, 1,301 rows 281 us against 286.)
 // K of the next chunk is loaded once this chunk's codes are converted, V likewise.  out = acc / max(l,
 // 1e-20) * sigmoid(gate), bf16.
 // What bounds it: the gather (528 bytes per cell, row and KV head, from the Infinity Cache where a context
@@ -932,7 +935,6 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a, int gr
 // rows over 2,048 of 33-41 thousand cells 3,400 -> 1,775 us (9.8 TB/s gathered), 1,301 rows over 2,048 of 9-10
 // thousand 530 -> 301 us.
 constexpr int AT_C = 32;                      // cells per wave and step
-constexpr float AT_LAZY = 6.0f;               // log2 units
 constexpr int AT_OLD = 256 + 4;               // LDS row stride of the partial outputs (floats)
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 
@@ -1066,7 +1068,7 @@ __global__ void __launch_bounds__(256, 2) pf_attn_kernel(PfAttn a) {
             if (16 * (e >> 2) + (e & 3) < left) mx = fmaxf(mx, z[e]);
         }
         mx = at_rows<true>(mx);
-        if (__any(mx > m_ref + AT_LAZY)) {
+        if (__any(mx > m_ref)) {
             const float m_new = fmaxf(m_ref, mx), al = __builtin_amdgcn_exp2f(m_ref - m_new);
             m_ref = m_new;
             l_sum *= al;
