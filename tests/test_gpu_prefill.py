@@ -511,6 +511,28 @@ def test_prefill_chunking_is_exact_small(wz, gpu):
         b.close()
 
 
+def test_prefill_chunking_is_exact_past_4_gib_of_channels(wz, gpu):
+    """64 + 64 delta-rule heads hold 98,304 bytes of channels a row: rows from 43,691 on lie past 2^32 bytes of a
+    chunk's first.  One chunk of 44,000 rows against two that stay below, two delta-rule layers (the second
+    layer's state depends on every output of the first)."""
+    print("case prefill_chunking_4_gib", flush=True)
+    B = 44000
+    cfg = pf_cfg(ctx_max=B + 8, n_layers=2)
+    cfg.gdn_hk = cfg.gdn_hv = 64
+    cfg.qsa_period = 4                                # no sparse-attention layer among the two
+    toks = [int(t) for t in np.random.default_rng(9).integers(0, cfg.n_vocab, B)]
+    a, ra = run_chunks(cfg, toks, [B])
+    try:
+        b, rb = run_chunks(cfg, toks, [B // 2, B // 2])
+        try:
+            assert_same_state(a, b, cfg, B)
+            assert np.array_equal(ra[-(B // 2):], rb)
+        finally:
+            b.close()
+    finally:
+        a.close()
+
+
 def baseline_cfg(n_layers, ctx_max, qsa_period=4):
     c = wzy_amd.StageCfg()
     wzy_amd.lib().wzy_stage_cfg_default(C.byref(c), ctx_max)

@@ -576,14 +576,22 @@ __global__ void __launch_bounds__(256) pf_gdn_recur_kernel(PfGdn g) {
     };
     // q does not go through LDS: a lane keeps its 4 q values of the 32 rows in registers and reloads a
     // row's right after its use, 32 rows ahead (four waves reading k and q of every row from LDS kept the
-    // LDS busier than the VALU).  Byte offsets stop at the last row.
-    const char* q_b = (const char*) (g.conv_out + (size_t) kh * 128);
-    const uint32_t q_step = (uint32_t) QKV * 4, q_last = (uint32_t) (g.B - 1) * q_step + r8 * 16;
-    uint32_t q_off = r8 * 16;
+    // LDS busier than the VALU).  A lane's offset counts from the first of 32 rows and stops at the chunk's
+    // last row; from the chunk's first row it would pass 32 bits (64 + 64 heads: at 43,691 rows).
+    const char* const q_b = (const char*) (g.conv_out + (size_t) kh * 128);
+    const uint32_t q_step = (uint32_t) QKV * 4;
+    const char* q_w;
+    uint32_t q_off, q_end;
+    auto q_rows = [&](int r0) {                             // the next 32 rows to load are r0 ..
+        r0 = min(r0, g.B - 1);
+        q_w = q_b + (size_t) r0 * q_step;
+        q_off = r8 * 16;
+        q_end = q_off + min(GR_STEPS - 1, g.B - 1 - r0) * q_step;
+    };
     f32x4_t q4[GR_STEPS];
     auto next_q = [&]() {
-        const f32x4_t v = *(const f32x4_t*) (q_b + q_off);
-        q_off = min(q_off + q_step, q_last);
+        const f32x4_t v = *(const f32x4_t*) (q_w + q_off);
+        q_off = min(q_off + q_step, q_end);
         return v;
     };
 
@@ -639,6 +647,7 @@ __global__ void __launch_bounds__(256) pf_gdn_recur_kernel(PfGdn g) {
     };
 
     const int nfull = g.B / GR_STEPS, rest = g.B - nfull * GR_STEPS;
+    q_rows(0);
 #pragma unroll
     for (int st = 0; st < GR_STEPS; ++st) q4[st] = next_q();
     load(0);
@@ -659,6 +668,7 @@ __global__ void __launch_bounds__(256) pf_gdn_recur_kernel(PfGdn g) {
     for (int kb = 0; kb < nfull; ++kb) {
         const int bb = kb & 1, t0 = kb * GR_STEPS;
         load(t0 + GR_STEPS);
+        q_rows(t0 + GR_STEPS);
         get(bb, 0);
         get(bb, 1);
 #pragma unroll
