@@ -164,8 +164,8 @@ int wzy_moe_prefill(const wzy_moe_weights* w, const float* x, int n_tok, float* 
  * its launch groups on `stream`; us_stages[8] = mean microseconds of
  *   0 x -> bf16, 1 router GEMM, 2 routing + shared gate, 3 expert tiles and entry lists,
  *   4 shared gate|up, 5 shared down, 6 routed gate|up, 7 routed down + per-token combine.
- * Chunks below 8,192 tokens run the shared expert inside the routed launches: groups 4 and 5 are then
- * empty and 6 and 7 include it.
+ * wzy_moe_prefill runs the launches of 4 and 5 inside those of 6 and 7; here each group is launched by itself,
+ * so the groups add up to more than a call takes.
  * Counterpart of the reference's WZY_PF_PROF phase timers (src/wzy_prefill_tc.cuh:734-741). */
 int wzy_moe_prefill_time(const wzy_moe_weights* w, const float* x, int n_tok, float* comb, void* workspace,
                          size_t workspace_bytes, int iters, float* us_stages, void* stream);

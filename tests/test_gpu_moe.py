@@ -611,6 +611,27 @@ def test_moe_prefill_time_entry(wz, gpu):
     np.testing.assert_array_equal(host(comb), comb0)
 
 
+@pytest.mark.parametrize("N", [3000, 8200])
+def test_moe_prefill_time_groups_hold_the_shared_expert(wz, gpu, N):
+    """The shared expert's groups time its launches at every chunk length: with one routed expert per token the
+    shared one does as much work, so its groups are of the routed ones' size (an empty group reads 4 or 5 us)."""
+    print("case moe_prefill_time_shared N=%d" % N, flush=True)
+    D, F, E, K = 1024, 512, 64, 1
+    m = mi.make_layer(wz, 6, 0, D, F, E, K, blobs=[])
+    w, keep = device_layer(wz, m)
+    x = mi.make_x(wz, 6, 0, N, D)
+    comb0, _, _ = run_gpu_prefill(wz, w, x, N)
+    xd, comb = dev(x), DA(N * D, np.float32)
+    nws = wz.wzy_moe_prefill_workspace_bytes(D, F, E, K, N)
+    ws = DA(nws, np.uint8)
+    us = (C.c_float * 8)()
+    wz.wzy_moe_prefill_time(C.byref(w), xd.ptr, N, comb.ptr, ws.ptr, nws, 5, us, None)
+    wz.wzy_device_sync()
+    print(" ".join("%.1f" % u for u in us), flush=True)
+    assert us[4] > 0.25 * us[6] and us[5] > 0.25 * us[7], list(us)
+    np.testing.assert_array_equal(host(comb), comb0)
+
+
 def test_moe_prefill_full_chunk_rows(wz, orc, gpu):
     """BASELINE config 5 at full size: one 8,192-token chunk through the BASELINE layer.  A token's
     output depends on its own row only (tiles mix tokens, sums do not), so sampled rows equal, bit for

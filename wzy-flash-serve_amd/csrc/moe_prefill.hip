@@ -12,7 +12,7 @@
 //   7. pf_expert<gate|up, NVFP4> routed, one expert tile per workgroup, SwiGLU -> act bf16 [N*K x F]
 //   8. pf_expert<down, NVFP4>    routed -> y fp32 [N*K x D] per entry; pf_combine: comb[t] +=
 //                  sum_k w_k * y[pos(t, k)] in slot order (no float atomics)
-// Shorter chunks run 5 in the launch of 7 and 6 in the launch of 8.
+// 5 runs in the launch of 7 and 6 in the launch of 8.
 // pf_expert: 8 waves, 256 weight rows per workgroup, up to 128 A rows; weights staged through LDS in
 // coalesced 64-byte pieces of a row and dequantised by each lane into its v_mfma_f32_32x32x16_bf16 B fragment
 // (e2m1 x e4m3 block scale is exact in bf16, the fp32 tensor scale goes onto the accumulators;
@@ -619,11 +619,6 @@ extern "C" size_t wzy_moe_prefill_workspace_bytes(int n_embd, int n_ff, int n_ex
 namespace {
 
 constexpr int PF_N_STAGES = 8;     // timing groups of pf_enqueue
-// Rows from which the shared expert has launches of its own.  Below, its few dense blocks run beside the
-// routed tiles (307 tokens: 58 + 50 us as launches of 12 and 16 workgroups, under 10 beside them; 6,000 tokens
-// 933 us apart, 907 together); from here on both take the same time.
-constexpr int PF_APART_ROWS = 8192;
-
 int pf_check(const wzy_moe_weights* w, int N) {
     WZY_REQUIRE(w, "wzy_moe_prefill: null weights");
     WZY_REQUIRE(w->router && w->sgate && w->experts && w->sh_gate_q && w->sh_gate_s && w->sh_up_q && w->sh_up_s &&
@@ -642,7 +637,11 @@ int pf_check(const wzy_moe_weights* w, int N) {
 }
 
 // The launch sequence; with `ev`, event i is recorded before launch group i and event PF_N_STAGES
-// after the last one.
+// after the last one.  The shared expert's dense blocks run in the launches of the routed tiles: beside them
+// they cost less than in launches of their own at every length and shape measured (512 experts top-10, n_embd
+// 2,048, apart -> together: 2,048 tokens 480 -> 455 us, 8,192 1,143 -> 1,128, 25,600 3,117 -> 3,057; n_embd 2,560
+// 8,192 1,680 -> 1,646; 64 experts top-4, n_embd 512, 2,048 tokens 98 -> 70).  Only with `ev` they are launched
+// apart, so that each group is timed by itself; the results are the same bits.
 int pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, const PfWs& ws, hipStream_t st,
                 hipEvent_t* ev) {
     const int D = w->n_embd, F = w->n_ff, E = w->n_exp, K = w->top_k;
@@ -696,7 +695,7 @@ int pf_enqueue(const wzy_moe_weights* w, const float* x, int N, float* comb, con
     rdn.tiles = ws.tiles; rdn.n_tiles = ws.n_tiles;
     rdn.a = ws.act; rdn.tok = nullptr; rdn.topk = K;
     rdn.y = ws.y; rdn.ld_out = D;
-    const bool apart = N >= PF_APART_ROWS;
+    const bool apart = ev != nullptr;
     const PfExpArgs none{};
     mark(4);
     if (apart) launch_expert<false>(ws.mt, none, 0, sgu, st);
