@@ -416,6 +416,26 @@ def test_stage_prefill_at_attention_chunk_edges(wz, orc, gpu):
         st.close()
 
 
+def test_trace_of_a_longer_chunk(wz, orc, gpu):
+    """The trace buffers and the workspace grow with the chunk: the copies of a chunk longer than every one before
+    it are all its own (its k, v and indexer key rows among them, check_appends)."""
+    print("case trace_growth", flush=True)
+    cfg = pf_cfg()
+    toks = [int(t) for t in np.random.default_rng(19).integers(0, cfg.n_vocab, 150)]
+    st = wzy_amd.Stage(cfg)
+    try:
+        st.load_synthetic(SEED, 0)
+        wz.wzy_stage_set_trace(st.h, 1)
+        st.prefill(0, toks[:50])
+        st.sync()
+        om = OracleModel(wz, st, cfg, SEED)
+        st.prefill(50, toks[50:])
+        st.sync()
+        check_chunk(wz, orc, st, om, cfg, 50, toks[50:], "chunk of 100 after one of 50")
+    finally:
+        st.close()
+
+
 class QsaDims(C.Structure):                       # csrc/wzy_qsa.h
     _fields_ = [(n, C.c_int) for n in ("qh", "kvh", "hd", "n_rot", "ih", "idim", "iblk", "topk", "ctx_max", "ring_cap",
                                        "sinks")] + [("eps", C.c_float), ("window", C.c_int), ("f16_above", C.c_int)]
@@ -754,8 +774,9 @@ def test_prefill_block_scores_do_not_depend_on_the_launch(wz, gpu, n_ctx, B):
             st.close()
 
     whole = scores([B])
-    for t, (x, y) in enumerate(zip(whole, scores([900, 700, B - 1600]))):
-        assert np.isfinite(x).all() and np.array_equal(x, y), t
+    for parts in ([900, 700, B - 1600], [700, 333, B - 1033]):      # the longest first; the longest last
+        for t, (x, y) in enumerate(zip(whole, scores(parts))):
+            assert np.isfinite(x).all() and np.array_equal(x, y), (parts, t)
 
 
 @pytest.mark.timeout(900)

@@ -230,7 +230,7 @@ struct wzy_stage {
         float *R = nullptr, *lo = nullptr, *inj_a = nullptr, *inj_f = nullptr, *mixed = nullptr;
         uint16_t *xn = nullptr, *loh = nullptr, *xh = nullptr;
         float *qkv = nullptr, *z = nullptr, *ab = nullptr, *conv_out = nullptr, *decay = nullptr, *beta = nullptr,
-              *kq = nullptr, *o = nullptr;
+              *o = nullptr;
         float *qg = nullptr, *kk = nullptr, *vv = nullptr, *idx_raw = nullptr, *q_idx = nullptr, *scores = nullptr;
         int *sel = nullptr, *cnt = nullptr;
         float *block = nullptr, *comb = nullptr;
@@ -243,13 +243,22 @@ struct wzy_stage {
         size_t wbf_elems = 0;
         int* pos8 = nullptr;        // [cap / 8 + 2]: p0 + 8 i
         int sc_rows = 0;            // rows per block-score pass
-        float* tr = nullptr;        // per-layer trace [n_layers][4][tr_rows][D] (while tracing)
-        int* tr_sel = nullptr;      // per QSA layer: selected cells [n_qsa][tr_rows][topk], counts
-        int* tr_cnt = nullptr;      // [n_qsa][tr_rows]
-        float* tr_sc = nullptr;     // block scores [n_qsa][tr_rows][max_b]
-        float* tr_kv = nullptr;     // rows the KV / indexer appends quantise: [n_qsa][tr_rows][kvd k | kvd v | idim]
-        int tr_rows = 0;
     } pf;
+    // copies of the last chunk (wzy_stage_set_trace); they outlive the workspace, which is laid out anew for a
+    // longer chunk
+    struct PfTrace {
+        int rows = 0;
+        float* out = nullptr;       // per layer [n_layers][4][rows][D]
+        int* sel = nullptr;         // per QSA layer: selected cells [n_qsa][rows][topk], counts
+        int* cnt = nullptr;         // [n_qsa][rows]
+        float* sc = nullptr;        // block scores [n_qsa][rows][max_b]
+        float* kv = nullptr;        // rows the KV / indexer appends quantise: [n_qsa][rows][kvd k | kvd v | idim]
+        void release() {
+            for (void* p : {(void*) out, (void*) sel, (void*) sc, (void*) kv})
+                if (p) (void) hipFree(p);
+            *this = PfTrace{};
+        }
+    } pft;
     bool pre_head_pf = false;       // the pre-head rows of the last call are the prefill's residual
     const float* pre_head_rows() const { return pre_head_pf ? pf.R : R[r_pre_head]; }
     int prefill_reserve(int B);
@@ -298,10 +307,7 @@ wzy_stage::~wzy_stage() {
         if (sl.jobs) (void) hipFree(sl.jobs);
     }
     if (pf.base) (void) hipFree(pf.base);
-    if (pf.tr) (void) hipFree(pf.tr);
-    if (pf.tr_sel) (void) hipFree(pf.tr_sel);
-    if (pf.tr_sc) (void) hipFree(pf.tr_sc);
-    if (pf.tr_kv) (void) hipFree(pf.tr_kv);
+    pft.release();
     for (auto& kv : graph_execs)
         if (kv.second) (void) hipGraphExecDestroy(kv.second);
     for (void* p : allocs) (void) hipFree(p);
@@ -1512,47 +1518,32 @@ __global__ void pf_pos_kernel(int* pos8, int p0, int n) {
 
 int wzy_stage::prefill_reserve(int B) {
     const wzy_stage_cfg& c = cfg;
-    if (trace && B > pf.tr_rows) {
+    if (trace && B > pft.rows) {
         WZY_HIP_TRY(hipStreamSynchronize(stream));
-        if (pf.tr) WZY_HIP_TRY(hipFree(pf.tr));
-        if (pf.tr_sel) WZY_HIP_TRY(hipFree(pf.tr_sel));
-        if (pf.tr_sc) WZY_HIP_TRY(hipFree(pf.tr_sc));
-        if (pf.tr_kv) WZY_HIP_TRY(hipFree(pf.tr_kv));
-        pf.tr_kv = nullptr;
-        pf.tr = nullptr;
-        pf.tr_sel = pf.tr_cnt = nullptr;
-        pf.tr_sc = nullptr;
+        for (const char* n : {"trace.pf", "trace.pf_sel", "trace.pf_cnt", "trace.pf_scores", "trace.pf_kv"})
+            tensors.erase({-1, std::string(n)});
+        pft.release();
         const size_t n = (size_t) c.n_layers * 4 * B * D;
-        WZY_HIP_TRY(hipMalloc((void**) &pf.tr, n * 4));
         const size_t nq = (size_t) std::max(n_qsa, 1), ns = nq * B * c.idx_topk;
-        WZY_HIP_TRY(hipMalloc((void**) &pf.tr_sel, (ns + nq * B) * 4));
-        pf.tr_cnt = pf.tr_sel + ns;
-        const size_t nsc = nq * B * (size_t) max_b;
-        WZY_HIP_TRY(hipMalloc((void**) &pf.tr_sc, nsc * 4));
-        reg(-1, "trace.pf_scores", pf.tr_sc, nsc * 4);
-        const size_t nkv = nq * B * (size_t) (2 * KVD + c.idx_dim);
-        WZY_HIP_TRY(hipMalloc((void**) &pf.tr_kv, nkv * 4));
-        reg(-1, "trace.pf_kv", pf.tr_kv, nkv * 4);
-        pf.tr_rows = B;
-        reg(-1, "trace.pf", pf.tr, n * 4);
-        reg(-1, "trace.pf_sel", pf.tr_sel, ns * 4);
-        reg(-1, "trace.pf_cnt", pf.tr_cnt, nq * B * 4);
+        const size_t nsc = nq * B * (size_t) max_b, nkv = nq * B * (size_t) (2 * KVD + c.idx_dim);
+        WZY_HIP_TRY(hipMalloc((void**) &pft.out, n * 4));
+        WZY_HIP_TRY(hipMalloc((void**) &pft.sel, (ns + nq * B) * 4));
+        WZY_HIP_TRY(hipMalloc((void**) &pft.sc, nsc * 4));
+        WZY_HIP_TRY(hipMalloc((void**) &pft.kv, nkv * 4));
+        pft.cnt = pft.sel + ns;
+        pft.rows = B;
+        reg(-1, "trace.pf", pft.out, n * 4);
+        reg(-1, "trace.pf_sel", pft.sel, ns * 4);
+        reg(-1, "trace.pf_cnt", pft.cnt, nq * B * 4);
+        reg(-1, "trace.pf_scores", pft.sc, nsc * 4);
+        reg(-1, "trace.pf_kv", pft.kv, nkv * 4);
     }
     if (B <= pf.cap) return WZY_OK;
     WZY_HIP_TRY(hipStreamSynchronize(stream));
     if (pf.base) {
         WZY_HIP_TRY(hipFree(pf.base));
         dev_bytes -= pf.bytes;
-        float* keep_tr = pf.tr;
-        int *keep_sel = pf.tr_sel, *keep_cnt = pf.tr_cnt;
-        float* keep_sc = pf.tr_sc;
-        const int keep_rows = pf.tr_rows;
         pf = PfWs{};
-        pf.tr = keep_tr;
-        pf.tr_sc = keep_sc;
-        pf.tr_sel = keep_sel;
-        pf.tr_cnt = keep_cnt;
-        pf.tr_rows = keep_rows;
     }
     const size_t b = (size_t) B, maxb = (size_t) max_b;
     const int sc_rows = std::min(B, PF_SCORE_ROWS);
@@ -1697,8 +1688,8 @@ int wzy_stage::enqueue_prefill(int p0, int B, float* us_parts) {
     QsaDims dm = qd;
     // trace copies (wzy_stage_set_trace): [layer][slot][row][D], slots mixed_a, block, mixed_f, comb
     auto tr = [&](int l, int slot, const float* src) -> int {
-        if (!trace || !pf.tr) return WZY_OK;
-        WZY_HIP_TRY(hipMemcpyAsync(pf.tr + (((size_t) l * 4 + slot) * pf.tr_rows) * D, src, (size_t) B * D * 4,
+        if (!trace || !pft.out) return WZY_OK;
+        WZY_HIP_TRY(hipMemcpyAsync(pft.out + (((size_t) l * 4 + slot) * pft.rows) * D, src, (size_t) B * D * 4,
                                    hipMemcpyDeviceToDevice, st));
         return WZY_OK;
     };
@@ -1753,9 +1744,9 @@ int wzy_stage::enqueue_prefill(int p0, int B, float* us_parts) {
             pa.q_norm = w.q_norm; pa.k_norm = w.k_norm; pa.iq_norm = w.idx_qn; pa.cos_tab = cos_tab; pa.sin_tab = sin_tab;
             pa.kv = w.kv;
             WZY_TRY(launch_pf_qsa_prep(pa, B, st));
-            if (trace && pf.tr_kv) {                 // k (after norm + RoPE), v and the raw indexer key rows
+            if (trace && pft.kv) {                 // k (after norm + RoPE), v and the raw indexer key rows
                 const size_t rw = 2 * (size_t) KVD + ID;
-                float* dst = pf.tr_kv + (size_t) w.local * pf.tr_rows * rw;
+                float* dst = pft.kv + (size_t) w.local * pft.rows * rw;
                 WZY_HIP_TRY(hipMemcpy2DAsync(dst, rw * 4, pf.kk, (size_t) KVD * 4, (size_t) KVD * 4, B,
                                              hipMemcpyDeviceToDevice, st));
                 WZY_HIP_TRY(hipMemcpy2DAsync(dst + KVD, rw * 4, pf.vv, (size_t) KVD * 4, (size_t) KVD * 4, B,
@@ -1775,8 +1766,8 @@ int wzy_stage::enqueue_prefill(int p0, int B, float* us_parts) {
                     sa.dm = dm; sa.pos = pf.pos8 + q0 / 8; sa.pooled = w.ix.pooled; sa.dead = w.ix.dead;
                     sa.q_idx = pf.q_idx + (size_t) q0 * IH * ID; sa.scores = pf.scores; sa.max_b = max_b;
                     WZY_TRY(launch_pf_scores(sa, qb, p0 + q0 + qb, st));
-                    if (trace && pf.tr_sc)
-                        WZY_HIP_TRY(hipMemcpyAsync(pf.tr_sc + ((size_t) w.local * pf.tr_rows + q0) * max_b, pf.scores,
+                    if (trace && pft.sc)
+                        WZY_HIP_TRY(hipMemcpyAsync(pft.sc + ((size_t) w.local * pft.rows + q0) * max_b, pf.scores,
                                                    (size_t) qb * max_b * 4, hipMemcpyDeviceToDevice, st));
                 }
                 const int max_n_kv = p0 + q0 + qb;
@@ -1790,10 +1781,10 @@ int wzy_stage::enqueue_prefill(int p0, int B, float* us_parts) {
                                                 std::min(WZY_MAX_W, qb - g0), st));
                 }
             }
-            if (trace && pf.tr_sel) {
-                WZY_HIP_TRY(hipMemcpyAsync(pf.tr_sel + (size_t) w.local * pf.tr_rows * c.idx_topk, pf.sel,
+            if (trace && pft.sel) {
+                WZY_HIP_TRY(hipMemcpyAsync(pft.sel + (size_t) w.local * pft.rows * c.idx_topk, pf.sel,
                                            (size_t) B * c.idx_topk * 4, hipMemcpyDeviceToDevice, st));
-                WZY_HIP_TRY(hipMemcpyAsync(pf.tr_cnt + (size_t) w.local * pf.tr_rows, pf.cnt, (size_t) B * 4,
+                WZY_HIP_TRY(hipMemcpyAsync(pft.cnt + (size_t) w.local * pft.rows, pf.cnt, (size_t) B * 4,
                                            hipMemcpyDeviceToDevice, st));
             }
             PfAttn at{};
