@@ -543,6 +543,22 @@ def test_moe_prefill_tile_sizes_agree(wz, gpu):
         np.testing.assert_array_equal(c, comb[:n * D])
 
 
+@pytest.mark.parametrize("skip", [1, 3, 7])
+def test_moe_prefill_gate_row_at_any_bf16(wz, gpu, skip):
+    """The shared-expert gate row, read 16 bytes at a time, may start at any bf16 of a buffer."""
+    print("case moe_prefill_gate_row +%d" % skip, flush=True)
+    D, F, E, K, N = 768, 128, 64, 4, 70
+    m = mi.make_layer(wz, 5, 0, D, F, E, K)
+    x = mi.make_x(wz, 5, 0, N, D)
+    w, keep = device_layer(wz, m)
+    comb, ids, wts = run_gpu_prefill(wz, w, x, N)
+    row = dev(np.concatenate([np.zeros(skip, np.int16), m.sgate.view(np.int16), np.zeros(8, np.int16)]))
+    w.sgate = row.ptr + 2 * skip
+    c, i, v = run_gpu_prefill(wz, w, x, N)
+    np.testing.assert_array_equal(i, ids)
+    np.testing.assert_array_equal(c, comb)
+
+
 def test_moe_prefill_rejects_bad_shapes(wz, gpu):
     D, F, E, K = 256, 128, 48, 4                  # 48 experts: not a multiple of 64
     m = mi.make_layer(wz, 1, 0, D, F, 64, K, blobs=[])

@@ -427,9 +427,10 @@ __global__ void __launch_bounds__(256) pf_route_kernel(const float* __restrict__
         p[i] = idx < E ? v : -INFINITY;
     }
     float s = 0.f;
-    for (int d = lane * 8; d < D; d += 512) {                    // D a multiple of 256: whole 16-byte pieces
-        const uint4 gv = *(const uint4*) (sgate + d), xv = *(const uint4*) (xb + (size_t) t * D + d);
-        const uint32_t ga[4] = {gv.x, gv.y, gv.z, gv.w}, xa[4] = {xv.x, xv.y, xv.z, xv.w};
+    // D a multiple of 256: whole 16-byte pieces; the caller's gate row may start at any bf16
+    typedef u32x4_t u32x4_any_t __attribute__((aligned(2)));
+    for (int d = lane * 8; d < D; d += 512) {
+        const u32x4_t ga = *(const u32x4_any_t*) (sgate + d), xa = *(const u32x4_t*) (xb + (size_t) t * D + d);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             s = fmaf(bf16_lo(ga[i]), bf16_lo(xa[i]), s);
