@@ -445,6 +445,16 @@ class PfAttn(C.Structure):                        # csrc/wzy_prefill.h
     _fields_ = [("dm", QsaDims)] + [(n, C.c_void_p) for n in ("pos", "qg", "kq", "ks", "vq", "vs", "sel", "out")]
 
 
+def run_attention(wz, dims, ptrs, rows):
+    """pf_attn_kernel on operands as they stand, which no entry point takes: bf16 bits [rows, heads, 256]"""
+    out = DA((rows, dims.qh, dims.hd), np.uint16)
+    arg = PfAttn(dims, *ptrs, out.ptr)
+    launch = C.CDLL(wz.path)["_ZN3wzy14launch_pf_attnERKNS_6PfAttnEiP12ihipStream_t"]
+    assert launch(C.byref(arg), rows, None) == 0
+    wz.wzy_device_sync()
+    return out.numpy()
+
+
 def test_attention_weights_keep_the_largest_exact(wz, gpu):
     """A softmax weight of 1 is exact in fp16, so the largest one adds no rounding of its own.  One wave sees a
     cell of weight 2^-3.6 to 2^-5.9 in its first chunk (with V = 0) and the largest in its second; every other
@@ -470,20 +480,42 @@ def test_attention_weights_keep_the_largest_exact(wz, gpu):
     d = [DA.from_numpy(np.ascontiguousarray(x).ravel()) for x in
          (np.array([n_kv - 1], np.int32), qg, kq, ks.view(np.uint16), vq, vs.view(np.uint16),
           np.arange(2048, dtype=np.int32))]
-    out = DA(heads * hd, np.uint16)
-    arg = PfAttn(dims, *[x.ptr for x in d], out.ptr)
-    # internal to the library: no entry point takes a query as it stands
-    launch = C.CDLL(wz.path)["_ZN3wzy14launch_pf_attnERKNS_6PfAttnEiP12ihipStream_t"]
-    assert launch(C.byref(arg), 1, None) == 0
-    wz.wzy_device_sync()
+    out = run_attention(wz, dims, [x.ptr for x in d], 1)
     v = (vq[hi].astype(np.float16) * np.repeat(vs[hi], 64)).astype(np.float64)
     want = v[None, :] / (1.0 + np.exp(-s.astype(np.float64)))[:, None]
     low = bits_to_f32((want.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)).astype(np.float64)
     tie = low + 2.0 ** (np.floor(np.log2(want)) - 8)                               # halfway to the next bf16
     sure = np.abs(want - tie) > want * 2.0 ** -19
     assert sure.mean() > 0.99
-    got = out.numpy().reshape(heads, hd)
-    np.testing.assert_array_equal(got[sure], bf16_bits(want)[sure])
+    np.testing.assert_array_equal(out[0][sure], bf16_bits(want)[sure])
+
+
+def test_attention_cells_past_4_gib(wz, gpu):
+    """Code planes above 2^32 bytes (more KV heads or cells than the usual models': 2^24 cells of one KV head, or a
+    million of sixteen) take the kernel's 64-bit offsets: rows that attend cells past that mark equal rows that
+    attend the same cells at the start of a small store."""
+    print("case attention_past_4_gib", flush=True)
+    heads, hd, rows, topk, far = 12, 256, 5, 2048, 1 << 24
+    rng = np.random.default_rng(4)
+    qg = DA.from_numpy(rng.standard_normal((rows, heads, 2, hd)).astype(np.float32))
+    cells = [rng.integers(-127, 128, (topk, hd)).astype(np.int8),
+             rng.uniform(2.0 ** -7, 2.0 ** -6, (topk, hd // 64)).astype(np.float16).view(np.uint16),
+             rng.integers(-127, 128, (topk, hd)).astype(np.int8),
+             rng.uniform(2.0 ** -7, 2.0 ** -6, (topk, hd // 64)).astype(np.float16).view(np.uint16)]
+    sel = np.stack([rng.permutation(topk) for _ in range(rows)]).astype(np.int32)
+    res = []
+    for base in (0, far):
+        n = base + topk + rows                                  # the rows' own cells come last and are not selected
+        dims = QsaDims(heads, 1, hd, 64, 4, 128, 4, topk, n, 0, 0, 1e-6, 0, 0)
+        store = [DA((n,) + c.shape[1:], c.dtype, zero=True) for c in cells]
+        for d, c in zip(store, cells):
+            wz.wzy_memcpy_h2d(d.ptr + base * c[0].nbytes, c.ctypes.data, c.nbytes, None)
+        pos, ids = DA.from_numpy(np.array([base + topk], np.int32)), DA.from_numpy(sel + base)
+        res.append(run_attention(wz, dims, [pos.ptr, qg.ptr] + [d.ptr for d in store] + [ids.ptr], rows))
+        for d in store:
+            d.free()
+    assert (res[0] != 0).any()
+    np.testing.assert_array_equal(res[0], res[1])
 
 
 def run_chunks(cfg, toks, splits, seed=SEED, n_ctx=0):
