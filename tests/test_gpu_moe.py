@@ -462,8 +462,8 @@ def bf16_round64(a):
     (256, 128, 64, 4, 1),          # one token, one partial row tile
     (256, 128, 64, 4, 130),        # ragged: 3 row tiles, the last of 2 rows
     (256, 128, 64, 8, 600),
-    (256, 128, 64, 8, 1100),       # ~137 entries per expert: one partly filled 256-entry tile each
-    (256, 128, 64, 8, 2100),       # ~262 entries per expert: about half span two 256-entry tiles
+    (256, 128, 64, 8, 1100),       # ~137 entries per expert: about three in four cut into two 128-entry tiles
+    (256, 128, 64, 8, 2100),       # ~262 entries per expert: two or three 128-entry tiles, cut equal
     (512, 256, 128, 6, 77),
     (256, 128, 64, 12, 300),       # K = 12: a full 8-slot combine pass, then a predicated one
     (256, 128, 128, 8, 1000),      # 16 router A tiles (XCD-grouped router blocks), the last of 40 rows
@@ -483,7 +483,7 @@ def test_moe_prefill_parity(wz, orc, gpu, D, F, E, K, N):
     logits = prefill_logits(m, x).ravel()
     exact = check_ids(orc, logits, E, K, N, ids, ids_o)
     assert exact >= N - max(1, N // 50), (exact, N)
-    if N * K > 256 * E:                 # the case meant to split experts over two tiles does so
+    if N * K > 256 * E:                 # the case meant to cut experts into three tiles does so
         assert np.bincount(ids_o, minlength=E).max() > 256
     rows = np.array([np.array_equal(ids[t * K:(t + 1) * K], ids_o[t * K:(t + 1) * K]) for t in range(N)])
     wr = np.repeat(rows, K)

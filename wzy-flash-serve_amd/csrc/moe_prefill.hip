@@ -34,7 +34,6 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 namespace {
 
@@ -72,7 +71,6 @@ WZY_DEV uint16_t f_to_bf16(float f) {                // hardware conversion, rou
 WZY_DEV uint32_t pack_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{a, b}, bf16x2_t));
 }
-WZY_DEV float bf16_bits_to_f(uint32_t h) { return __builtin_bit_cast(float, h << 16); }
 WZY_DEV uint32_t f_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
 
 // MFMA B fragment (8 consecutive k of one weight row) from one 16-value NVFP4 sub-block: bytes
@@ -563,8 +561,12 @@ struct PfWs {
 // Entries per expert tile.  Both sizes put two workgroups on a CU, so that one computes while the other waits
 // for a K step (one workgroup a CU with 256-entry tiles: 307 tokens 324 + 179 us gate|up + down, now 212 +
 // 116; 8,192 tokens 490 + 533, now 483 + 512).  64-entry tiles stage half the rows and load two steps ahead;
-// beyond 60 entries an expert too many experts need two of them (512 experts top-10, whole block: 59 entries
-// 565 us with 64 against 592 with 128, 68 entries 650 against 632).
+// near 60 entries an expert too many experts need two of them.  Whole block with 64 against 128: 512 experts
+// top-10, n_embd 2,048, 50 entries 506 and 515 us, 57.5 548 and 549, 62.5 610 and 563; n_embd 2,560, n_ff 640, 50
+// entries 741 and 769, 57.5 821 and 807, 62.5 890 and 834; 128 experts top-8, 56 entries 175 and 182, 64 195 and
+// 195.  (64 experts of n_embd 512 leave the chip idle either way: 75 entries 57 and 66.)  The 128-entry kernel
+// fills its 128 registers; its loops over four row blocks reload one register of routed gate|up every two chunks
+// and two of the shared down from scratch, beside 64 and 32 MFMAs.
 int pf_tile_entries(size_t n_ent, int E) { return n_ent <= (size_t) 60 * E ? 64 : 128; }
 
 PfWs pf_ws_carve(void* base, size_t cap, int D, int F, int E, int K, int N, size_t* need) {

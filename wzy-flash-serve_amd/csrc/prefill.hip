@@ -75,7 +75,7 @@ WZY_DEV uint4 q8_quarter_bf16(uint32_t a, uint32_t b, float sc) {
 // registers allow no more); the next k step still loads into registers during the MFMAs, and a second
 // barrier per step guards the buffer.  Launches with at least 512 tiles use it; smaller ones keep two.
 // With a thread's 64 bytes of one row per step replaced by whole rows per eight lanes (below), 8,192 x 6,144 x
-// 2,048 took 338 -> 275 us from Q8_0 and 295 -> 260 us from bf16 (791 TFLOP/s), 250 x 12,288 x 2,048 53 -> 31.
+// 2,048 took 296 -> 261 us from Q8_0 and 276 -> 250 us from bf16 (826 TFLOP/s), 250 x 12,288 x 2,048 50 -> 29.
 template <int T, bool UM, bool SB, bool Q8>
 __global__ void __launch_bounds__(256, SB ? (UM ? 3 : 4) : T == 64 ? (Q8 ? 4 : 3) : 2) pf_gemm_kernel(GemmArgs ga) {
     constexpr int GM = T, GN = T, NB = T / 64;                     // tile; 32 x 32 blocks per wave and side
@@ -484,19 +484,11 @@ __global__ void __launch_bounds__(256) pf_gdn_hist_kernel(PfGdn g) {
     h[2] = v[2];
 }
 
-// Sum over each 32-lane half: the 16-lane DPP sum, then the two rows of the half swapped in one
-// VALU op (v_permlane16_swap) and added; every lane of the half gets the same value.
-// (Written as inline assembly: through the builtin, this compiler hands both results of the swap in
-// one register when they feed one add.  The s_nops cover the VALU-write-to-permlane hazard.)
-WZY_DEV float sum32_pl(float v) {
-    v = sum16(v);
-    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-    return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
-}
 // Sums of 32 per-lane values over each 32-lane half, transposed: lane r of the half returns the sum of
 // v[r].  Five partner levels, each splitting the values a lane holds in two (16 swaps + 16 adds, then
 // reduce_level's 3 operations per value left): about 2.4 operations per value instead of 7.
+// (The swap is inline assembly: through the builtin, this compiler hands both results of the swap in
+// one register when they feed one add.  The s_nops cover the VALU-write-to-permlane hazard.)
 WZY_DEV float sum32_t(const float (&v)[32]) {
     const int lane = threadIdx.x & 63;
     float b[16], c[8], d[4], e[2], f[1];
@@ -534,7 +526,7 @@ static_assert(GR_STEPS == GR_LPC, "one output row per lane of a column");
 // and no k . q correction).  k and, per column, v with the row's decay and beta go through LDS 32 rows at a
 // time in 16-byte pieces, the next 32 loaded while these run; q stays out of LDS.
 // 8,192 rows x 16 heads: 1,050 us with both sums reduced per row and k, q, v through LDS; 861 with the
-// transposed sum and reads two rows ahead; 784 with q in registers (about 32 instructions a row, of which
+// transposed sum and reads two rows ahead; about 800 with q in registers (about 32 instructions a row, of which
 // 13 form the chain through kv).
 // (pf_gdn_recur_kh_kernel, src/wzy_qsa_wmma.cuh:56-195; fused_gdn_step_norm_multi,
 // src/wzy_kernels_v2.cuh:908-984)
@@ -942,8 +934,8 @@ __global__ void __launch_bounds__(256, 3) pf_score_kernel(QsaScoreArgs a, int gr
 // What bounds it: the gather (528 bytes per cell, row and KV head, from the Infinity Cache where a context
 // exceeds the L2) and about 480 VALU operations per 32 cells and wave for the conversions.  Against the
 // kernel before it, which staged K and a transposed V through LDS with three barriers per 64 cells: 8,192
-// rows over 2,048 of 33-41 thousand cells 3,400 -> 1,775 us (9.8 TB/s gathered), 1,301 rows over 2,048 of 9-10
-// thousand 530 -> 301 us.
+// rows over 2,048 of 33-41 thousand cells 3,260 -> 1,831 us (9.7 TB/s gathered), 1,300 rows over 2,048 of 9-10
+// thousand 530 -> 325 us.
 constexpr int AT_C = 32;                      // cells per wave and step
 constexpr int AT_OLD = 256 + 4;               // LDS row stride of the partial outputs (floats)
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
@@ -964,7 +956,7 @@ WZY_DEV f16x8_t at_k8(uint32_t a, uint32_t b, f16x2_t sc) {
     b ^= 0x80808080u;
     return at_join(at_lo(a) * sc, at_hi(a) * sc, at_lo(b) * sc, at_hi(b) * sc);
 }
-// maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (inline assembly as in sum32_pl)
+// maximum / sum over lanes l, l ^ 16, l ^ 32, l ^ 48 (inline assembly as in sum32_t)
 template <bool MAX>
 WZY_DEV float at_rows(float v) {
     uint32_t x = __builtin_bit_cast(uint32_t, v), y = x;
