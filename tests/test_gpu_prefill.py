@@ -563,6 +563,23 @@ def test_prefill_chunking_is_exact_small(wz, gpu):
         b.close()
 
 
+@pytest.mark.parametrize("splits", [[32, 32, 33], [1, 96], [31, 34, 32], [65, 32]])
+def test_prefill_chunking_is_exact_at_recurrence_buffer_edges(wz, gpu, splits):
+    """97 rows (three buffers of the delta rule's 32 rows and one row) against chunks that end before, at and after
+    a buffer: a row's bits do not depend on its place in one."""
+    print("case prefill_chunking_edges %s" % splits, flush=True)
+    cfg = pf_cfg()
+    toks = [int(t) for t in np.random.default_rng(13).integers(0, cfg.n_vocab, 97)]
+    a, ra = run_chunks(cfg, toks, [97])
+    b, rb = run_chunks(cfg, toks, splits)
+    try:
+        assert_same_state(a, b, cfg, 97)
+        assert np.array_equal(ra[-splits[-1]:], rb)
+    finally:
+        a.close()
+        b.close()
+
+
 def test_prefill_chunking_is_exact_past_4_gib_of_channels(wz, gpu):
     """64 + 64 delta-rule heads hold 98,304 bytes of channels a row: rows from 43,691 on lie past 2^32 bytes of a
     chunk's first.  One chunk of 44,000 rows against two that stay below, two delta-rule layers (the second
