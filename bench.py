@@ -56,7 +56,8 @@ PF_STAGES = ("x_to_bf16", "router_gemm", "route", "tiles", "shared_gate_up", "sh
 
 def prefill_moe(wz, st, n_tok, iters, seed):
     """Config-5 chunked-prefill MoE on layer 0 of the loaded stage: n_tok rows of N(0,1) x, every
-    launch group timed with HIP events (wzy_moe_prefill_time)."""
+    launch group timed with HIP events (wzy_moe_prefill_time, which launches the shared expert's groups
+    by themselves: a wzy_moe_prefill call, with them beside the routed ones, takes less than the sum)."""
     import numpy as np
     import wzy_amd
     w = wzy_amd.MoeWeights()
